@@ -93,10 +93,14 @@ static int emit_kind(const hb_desc& d, Emitted* e) {
             if (!d.wm || !d.wn || d.wm * d.wn > 16 || d.bm % (d.wm * d.mfma) ||
                 d.bn % (d.wn * d.mfma))
                 return fail(HB_ERR_UNSUPPORTED, "gemm: tile not a multiple of waves x mfma");
-            if (swi && (d.bn / (d.wn * d.mfma)) % 2)
+            bool experts = d.rows_of != HB_ROWS_DENSE;
+            // The gate and up sums meet in the LDS epilogue (dense rows,
+            // direct-to-LDS, whole 16-byte chunks of features), else in the
+            // wave's registers.
+            if (swi && (experts || !d.lds_dma || d.n % 8) && (d.bn / (d.wn * d.mfma)) % 2)
                 return fail(HB_ERR_UNSUPPORTED,
                             "gemm_swiglu: an even count of W fragments per wave (bn / (wn * mfma))");
-            bool experts = d.rows_of != HB_ROWS_DENSE;
+            if (swi && d.ksplit > 1) return fail(HB_ERR_UNSUPPORTED, "gemm_swiglu: no split K");
             if (experts && (!d.top_k || !d.experts || !d.tiles))
                 return fail(HB_ERR_INVALID, "gemm over experts: top_k, experts and tiles");
             e->threads = 64 * d.wm * d.wn;
@@ -124,7 +128,7 @@ static int emit_kind(const hb_desc& d, Emitted* e) {
             if (d.w_nt > 1 || (d.w_nt && !d.lds_dma))
                 return fail(HB_ERR_UNSUPPORTED, "gemm: w_nt with direct-to-LDS staging");
             if (d.sched > 3) return fail(HB_ERR_INVALID, "gemm: sched 0..3");
-            if (d.sched && (swi || experts || !d.lds_dma || d.dbuf < 2 || d.w_nt ||
+            if (d.sched && (experts || (swi && d.n % 8) || !d.lds_dma || d.dbuf < 2 || d.w_nt ||
                             d.wm * d.wn != (d.sched == 3 ? 4u : 8u) ||
                             ((d.bm * d.bk / 8) % 64) || ((d.bn * d.bk / 8) % 64) ||
                             (d.sched == 3 && (d.k / d.bk) % 2) ||

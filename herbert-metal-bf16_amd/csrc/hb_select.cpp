@@ -320,12 +320,31 @@ const Form kSplitForms[] = {
     {"pp_t256x256_ks4", 256, 256, 32, 4, 2, 16, 3, 1, 1, 0, 1, 4},
 };
 // The fused [gate | up] + SwiGLU forms (gate_up_pipes, qwen.rs:2148-2193):
-// bn W rows per tile = bn/2 features.
+// bn W rows per tile = bn/2 features.  The first is the one pf.fswi=1 names.
+// The ping-pong ones are the same tiles as the GEMM's: the SwiGLU from the
+// tile staged in LDS costs 2-4 us of a 2048 x 18432 x 2560 launch, where the
+// pass over the written [gate | up] rows costs 20-22 (256 x 288: 162.7 us
+// against 158.9 + 20.2; 512 rows, 256 x 160: 51.9 against 50.7 + 7.3).  The
+// narrow last ones are for short prompts, one row tile of 64 or 128 rows:
+// enough column tiles to reach every CU (230 of 80 W rows at 2 x 9216), and
+// 128 K a stage so that each barrier covers twice the loads (64 rows: 23.3 us
+// against 27.6 for the best unfused form and its pass).
 const Form kFusedForms[] = {
     {"fused128x64", 128, 128, 64, 2, 2, 16, 1, 1, 1},
     {"fused128x64b2", 128, 128, 64, 2, 2, 16, 1, 1, 0, 2},
     {"fused256x96", 256, 192, 64, 4, 2, 16, 1, 1, 1},
     {"fused256x128", 256, 256, 64, 4, 2, 32, 1, 1, 1},
+    {"fused256x144_pp_b4", 256, 288, 32, 4, 2, 16, 3, 1, 1, 4, 1},
+    {"fused256x128_pp_b4", 256, 256, 32, 4, 2, 16, 3, 1, 1, 4, 1},
+    {"fused256x96_pp", 256, 192, 32, 4, 2, 16, 3, 1, 1, 0, 1},
+    {"fused256x80_pp", 256, 160, 64, 4, 2, 16, 2, 1, 1, 0, 1},
+    {"fused256x80_pp_b4", 256, 160, 64, 4, 2, 16, 2, 1, 1, 4, 1},
+    {"fused128x80_pp", 128, 160, 64, 4, 2, 16, 3, 1, 1, 0, 1},
+    {"fused128x96_w8_s4", 128, 192, 64, 2, 4, 16, 3, 1, 0},
+    {"fused128x80_s4", 128, 160, 64, 4, 1, 16, 3, 1, 1},
+    {"fused128x40_s4", 128, 80, 64, 4, 1, 16, 3, 1, 1},
+    {"fused64x40_k128", 64, 80, 128, 4, 1, 16, 2, 1, 1},
+    {"fused64x48_s4", 64, 96, 64, 2, 2, 16, 3, 1, 1},
 };
 
 hb_desc form_desc(const Form& f, uint32_t k, uint32_t n, uint32_t out, bool mf) {

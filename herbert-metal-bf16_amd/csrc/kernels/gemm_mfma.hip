@@ -48,8 +48,10 @@
 // the SwiGLU in one (prefill.rs:755-824, gemm_nax_swiglu; for the experts,
 // the grouped gate|up and swiglu_slots, qwen_kernels.rs:2087-2117).  N is the
 // feature count nf and W holds 2*nf rows per expert (gate rows, then their
-// up rows); a tile covers BN/2
-// features: each wave's W fragments 0..IN/2-1 are gate rows and fragments
+// up rows); a tile covers BN/2 features.  Dense rows through direct-to-LDS
+// stages: the tile's gate rows, then its up rows, which meet in the LDS
+// epilogue (gemm_epi.h).  Otherwise in registers:
+// each wave's W fragments 0..IN/2-1 are gate rows and fragments
 // IN/2.. the up rows of the same features, so a lane holds the gate and the
 // up sums of the same outputs and writes h = rne(g * sigmoid(g) * u) with g,
 // u the bf16-rounded sums -- the bits of the unfused GEMM (same tile form)
@@ -104,8 +106,7 @@ static_assert(BK % KS == 0 && (CH & (CH - 1)) == 0, "K step");
 static_assert(NT % CH == 0, "threads a multiple of the chunks of a row");
 static_assert(NS >= 1 && NS <= 4, "1 to 4 stages");
 static_assert(HB_DMA || NS <= 2, "register staging: 1 or 2 stages");
-static_assert(!SWI || (IN % 2 == 0 && OUT == 0 && ROWS != 2),
-              "fused SwiGLU: dense or gathered rows, bf16 out, an even count of W fragments per wave");
+static_assert(!SWI || (OUT == 0 && ROWS != 2), "fused SwiGLU: dense or gathered rows, bf16 out");
 
 typedef __attribute__((ext_vector_type(FM == 16 ? 4 : 16))) float acc_t;
 
@@ -160,7 +161,9 @@ HB_DEV void store4(void* Yv, u64 at, float v0, float v1, float v2, float v3) {
 
 #include "gemm_epi.h"
 // Dense rows through direct-to-LDS stages: the epilogue through LDS.
-constexpr bool EPI_VIA_LDS = EPI_LDS && HB_DMA && ROWS == 0 && !SWI;
+constexpr bool EPI_VIA_LDS = EPI_LDS && HB_DMA && ROWS == 0;
+static_assert(!SWI || EPI_VIA_LDS || IN % 2 == 0,
+              "fused SwiGLU in registers: an even count of W fragments per wave");
 
 #define HB_INLINE __attribute__((always_inline))
 
@@ -265,6 +268,7 @@ extern "C" __global__ __launch_bounds__(NT) void HB_NAME(
     };
     auto w_row = [&](u32 r) HB_INLINE -> u32 {
         if (r >= BN) r = BN - 1;
+        if constexpr (SWI && EPI_VIA_LDS) return swi_w_row(n0, r);
         if constexpr (SWI) {
             // Tile row r: wave r / TN, its fragment i; gate rows for i <
             // IN/2, else the up rows of fragment i - IN/2's features.
@@ -528,12 +532,13 @@ extern "C" __global__ __launch_bounds__(NT) void HB_NAME(
                     if (f < N) {
                         const acc_t& g = acc[i][j];
                         const acc_t& u = acc[i + IN / 2][j];
-                        float h[4];
+                        float gr[4], ur[4], h[4];
 #pragma unroll
                         for (u32 e = 0; e < 4; e++) {
-                            const float gr = round_bf16(g[4 * q + e]), ur = round_bf16(u[4 * q + e]);
-                            h[e] = (gr * hb_sigmoid(gr)) * ur;
+                            gr[e] = round_bf16(g[4 * q + e]);
+                            ur[e] = round_bf16(u[4 * q + e]);
                         }
+                        swiglu_n<4>(gr, ur, h);
                         store4(Yv, (u64)yrow * N + f, h[0], h[1], h[2], h[3]);
                     }
                 }

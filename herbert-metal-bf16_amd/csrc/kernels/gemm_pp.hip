@@ -66,7 +66,8 @@
 // HB_GRP (ping-pong: which waves form a group: 0 waves 0-3 / 4-7, 1 even /
 // odd waves), HB_KSPLIT (s > 1: K cut into s parts, part p's f32 sums into
 // slab p of Y, [m_launch][N] floats each, as in gemm_mfma.hip; a second
-// kernel adds the slabs).
+// kernel adds the slabs), HB_SWIGLU 1 (N features, W [gate (N) | up (N)]: the
+// SwiGLU of the sums in the epilogue, gemm_epi.h).
 //
 // Bindings: state (u32[4], state[3] = rows), W, X, Y, list, tiles (unused:
 // dense rows); then the rows the launch was sized for (m_launch).
@@ -92,7 +93,12 @@ constexpr u32 S = BK / KS;                 // MFMA steps per K tile
 constexpr u32 KSP = HB_KSPLIT;
 constexpr u32 KT = K / BK / KSP;           // K tiles of one part
 constexpr u32 NS = HB_STAGES;
-constexpr u32 NTILES = (N + BN - 1) / BN;
+#ifndef HB_SWIGLU
+#define HB_SWIGLU 0
+#endif
+constexpr bool SWI = HB_SWIGLU != 0;
+constexpr u32 BF = SWI ? BN / 2 : BN;      // output columns of a tile
+constexpr u32 NTILES = (N + BF - 1) / BF;
 constexpr u32 XST = BM * CH, WST = BN * CH;  // chunks per stage
 // Wave-loads (64 chunks, 1 KiB) per stage of each operand, shared out over
 // the NWV waves: wave w issues the operand's wave-loads w, w + NWV, ...; when
@@ -112,6 +118,8 @@ static_assert(WM * WN == NWV, "eight wavefronts (ping-pong) or four");
 static_assert(K % (BK * KSP) == 0, "K a multiple of the K step times the parts");
 static_assert(KSP == 1 || OUT == 1, "split K: f32 partial sums");
 static_assert(N % 4 == 0, "N a multiple of 4");
+static_assert(!SWI || (OUT == 0 && KSP == 1 && N % 8 == 0 && BN % 16 == 0),
+              "fused SwiGLU: bf16 out, no split, whole 16-byte chunks of features");
 static_assert(TM % FM == 0 && TN % FM == 0, "wave tile a multiple of the MFMA block");
 static_assert(BK % KS == 0 && (CH & (CH - 1)) == 0, "K step");
 static_assert(XST % 64 == 0 && WST % 64 == 0, "whole wave-loads per stage");
@@ -209,7 +217,7 @@ extern "C" __global__ __launch_bounds__(NT) void HB_NAME(
     if (gm >= mb || gn >= NTILES) return;
     const u32 row0 = gm * BM;
     const u32 rows = m - row0 < BM ? m - row0 : BM;
-    const u32 n0 = gn * BN;
+    const u32 n0 = gn * BF;
 
     // This wave's wave-loads of a stage: LDS slot p = q*64 + lane of the
     // operand's stage holds (row p / CH, chunk (p % CH) ^ swizzle(row));
@@ -227,8 +235,8 @@ extern "C" __global__ __launch_bounds__(NT) void HB_NAME(
     for (u32 i = 0; i < WLMAX; i++) {
         const u32 p = (wave + NWV * i) * 64 + lane, r = p / CH;
         const u32 cc = (p % CH) ^ ((r >> HB_SWZ) & (CH - 1));
-        const u32 n = n0 + r;
-        woff[i] = ((n < N ? n : N - 1) * K + part * (KT * BK) + cc * 8) * 2;
+        const u32 n = SWI ? swi_w_row(n0, r) : n0 + r < N ? n0 + r : N - 1;
+        woff[i] = (n * K + part * (KT * BK) + cc * 8) * 2;
     }
 
     const __amdgpu_buffer_rsrc_t rX =

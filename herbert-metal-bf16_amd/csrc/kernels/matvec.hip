@@ -236,11 +236,7 @@ extern "C" __global__ __launch_bounds__(NT) void HB_NAME(const u16* __restrict__
 #if HB_XSRC == 1
         const u32x4 g = *(const u32x4*)(x + (u64)jj * 2 * K + off);
         const u32x4 u = *(const u32x4*)(x + (u64)jj * 2 * K + K + off);
-        u32x4 h;
-#pragma unroll
-        for (u32 e = 0; e < 4; e++)
-            h[e] = pack_bf16x2(swiglu1(bf16_lo(g[e]), bf16_lo(u[e])), swiglu1(bf16_hi(g[e]), bf16_hi(u[e])));
-        return h;
+        return swiglu_pairs(g, u);
 #else
         return *(const u32x4*)(x + (u64)jj * K + off);
 #endif

@@ -346,17 +346,7 @@ extern "C" __global__ __launch_bounds__(256) void HB_NAME(const u32x4* __restric
     const u64 i = (u64)blockIdx.x * 256 + threadIdx.x;
     if (i >= (u64)rows * CELLS) return;
     const u32 s = (u32)(i / CELLS), c = (u32)(i % CELLS);
-    const u32x4 g = gu[(u64)s * 2 * CELLS + c], u = gu[(u64)s * 2 * CELLS + CELLS + c];
-    u32x4 o;
-#pragma unroll
-    for (u32 e = 0; e < 4; e++) {
-        const float g0 = bf16_lo(g[e]), g1 = bf16_hi(g[e]);
-        const float u0 = bf16_lo(u[e]), u1 = bf16_hi(u[e]);
-        const float h0 = (g0 * hb_sigmoid(g0)) * u0;
-        const float h1 = (g1 * hb_sigmoid(g1)) * u1;
-        o[e] = pack_bf16x2(h0, h1);
-    }
-    h[i] = o;
+    h[i] = swiglu_pairs(gu[(u64)s * 2 * CELLS + c], gu[(u64)s * 2 * CELLS + CELLS + c]);
 }
 
 #elif HB_OP == 6

@@ -20,6 +20,15 @@ FUSED = {
     "fused256x128": dict(bm=256, bn=256, bk=64, wm=4, wn=2, mfma=32, dbuf=1, lds_dma=1, order=1),
     "fused64x32_reg": dict(bm=64, bn=64, bk=32, wm=1, wn=2, mfma=16, dbuf=0, lds_dma=0, order=0),
 }
+# The gate and up rows meeting in the LDS epilogue: the ping-pong tiles, odd
+# counts of W fragments per wave, more row tiles or features than the block.
+LDS_FUSED = {
+    "pp256x144": dict(bm=256, bn=288, bk=32, wm=4, wn=2, mfma=16, dbuf=3, lds_dma=1, order=1, band=4, sched=1),
+    "pp256x80": dict(bm=256, bn=160, bk=64, wm=4, wn=2, mfma=16, dbuf=2, lds_dma=1, order=1, sched=1),
+    "pp128x80": dict(bm=128, bn=160, bk=64, wm=4, wn=2, mfma=16, dbuf=3, lds_dma=1, order=1, sched=1),
+    "s4_128x40": dict(bm=128, bn=80, bk=64, wm=4, wn=1, mfma=16, dbuf=3, lds_dma=1, order=1),
+    "k128_64x40": dict(bm=64, bn=80, bk=128, wm=4, wn=1, mfma=16, dbuf=2, lds_dma=1, order=1),
+}
 APART = dict(bm=128, bn=128, bk=64, wm=2, wn=2, mfma=16, dbuf=1, lds_dma=1, order=1)
 
 
@@ -86,6 +95,52 @@ def test_fused_swiglu_equals_gemm_then_swiglu(gpu, form, m, k, nf):
     assert np.array_equal(h_fused, h_apart), "%s: fused != GEMM then SwiGLU" % form
     check_close(gu, orc.gemm(x, w), k, abs_products(x, w), "gate|up %s" % form)
     assert np.array_equal(h_apart, orc.swiglu(gu, nf))
+
+
+@pytest.mark.parametrize("form", sorted(LDS_FUSED))
+@pytest.mark.parametrize("m,k,nf", [(1, 256, 8), (57, 512, 200), (257, 256, 296)])
+def test_lds_fused_swiglu_equals_gemm_then_swiglu(gpu, form, m, k, nf):
+    """As above for the forms whose gate and up sums meet in LDS: equal bits
+    (the 16x16 MFMA's K order), at one row, a ragged tile and one row past
+    the tile, and feature counts below, at and past a tile's."""
+    x, w = inputs(m, k, nf, 0x5EED0007)
+    b = Bufs(gpu, x, w, m)
+    try:
+        b.fused(gpu.pipeline(hb.gemm_mma_swiglu(k, nf, **LDS_FUSED[form])), m)
+        h_fused = b.get("h")
+        b.gemm(gpu.pipeline(hb.gemm_mma(k, 2 * nf, 0, **APART)), m)
+        gu = b.get("gu")
+    finally:
+        b.free()
+    check_close(gu, orc.gemm(x, w), k, abs_products(x, w), "gate|up %s" % form)
+    assert np.array_equal(h_fused, orc.swiglu(gu, nf))
+
+
+def test_swiglu_every_gate(gpu):
+    """Every bf16 gate that is no NaN, alone among ordinary ones and beside
+    its neighbours, against the oracle's exp and division, bit for bit; a NaN
+    gate gives a NaN."""
+    bits = np.arange(65536, dtype=np.uint32).astype(np.uint16)
+    ks = gpu.pipeline(hb.swiglu_rows(8))
+    for u in (0x3F80, 0xC049, 0x0001, 0x7F7F):
+        alone = np.full((65536, 16), 0x3F80, np.uint16)
+        alone[:, 3] = bits
+        beside = np.concatenate([bits.reshape(8192, 8), np.full((8192, 8), 0x3F80, np.uint16)], axis=1)
+        for gu in (alone, beside):
+            gu = gu.copy()
+            gu[:, 8:] = u
+            a, h = gpu.alloc_with(gu), gpu.alloc(gu.nbytes // 2)
+            try:
+                gpu.launch(ks, [hb.r(a), hb.r(h)], gu.shape[0])
+                gpu.sync()
+                got = gpu.download(h, np.uint16, gu.size // 2).reshape(-1, 8)
+            finally:
+                gpu.free(a)
+                gpu.free(h)
+            want = orc.swiglu(gu, 8)
+            bad = (gu[:, :8] & 0x7FFF) > 0x7F80
+            assert np.array_equal(got[~bad], want[~bad])
+            assert np.all((got[bad] & 0x7FFF) > 0x7F80)
 
 
 def test_fused_swiglu_state_rows(gpu):
