@@ -110,6 +110,32 @@ HB_DEV u32x4 swiglu_pairs(u32x4 gv, u32x4 uv) {
     return o;
 }
 
+// The 64 lanes' sum in the xor butterfly's association (lanes 32 apart
+// first, then 16, 8, 4, 2, 1), every lane with the same bits: the halves and
+// the 16-lane rows by lane swaps, then rotations within 16 lanes (once lanes
+// 8 apart agree, a rotation by 4 holds what lane l ^ 4 does) and quads.  Six
+// __shfl_xor give the same value in six LDS-crossbar round trips.
+HB_DEV float butterfly_sum(float v) {
+    // Words by value: this compiler's __builtin_bit_cast of a vector's
+    // element takes element 0 whatever the index.
+    auto f32 = [](u32 w) { return __builtin_bit_cast(float, w); };
+    u32 b = __builtin_bit_cast(u32, v);
+    const auto h = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    v = f32(h[0]) + f32(h[1]);
+    b = __builtin_bit_cast(u32, v);
+    const auto q = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    v = f32(q[0]) + f32(q[1]);
+#define HB_DPP_ADD(ctrl)                                                                             \
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, \
+                                                               0xf, 0xf, true))
+    HB_DPP_ADD(0x128);  // row_ror:8
+    HB_DPP_ADD(0x124);  // row_ror:4
+    HB_DPP_ADD(0x4E);   // quad_perm [2,3,0,1]
+    HB_DPP_ADD(0xB1);   // quad_perm [1,0,3,2]
+#undef HB_DPP_ADD
+    return v;
+}
+
 // The row count of a block: state[3] as the reference's kernels read it
 // (src/metal/kernels.rs:15, prefill.rs:21-24), never more than the rows the
 // launch was sized for.

@@ -142,13 +142,6 @@ struct HbTrue { static constexpr bool value = true; };
 struct HbFalse { static constexpr bool value = false; };
 #define HB_INLINE2 __attribute__((always_inline))
 
-HB_DEV float wave_sum(float v) {
-    // Butterfly over the 64 lanes (xor 32, 16, ..., 1).
-#pragma unroll
-    for (int s = 32; s >= 1; s >>= 1) v += __shfl_xor(v, s, 64);
-    return v;
-}
-
 // The 64 lanes' sum of the matvec's row sums without the LDS crossbar:
 // pairs (quad_perm 1,0,3,2), quads (2,3,0,1), then the half-row and row
 // mirrors (once each 4- and 8-lane group is uniform, the mirrored lane
@@ -207,7 +200,7 @@ extern "C" __global__ __launch_bounds__(NT) void HB_NAME(const u16* __restrict__
                 const float v = bf16_to_f32(x[(u64)jj * K + tid + i * 256]);
                 a = __builtin_fmaf(v, v, a);
             }
-            a = wave_sum(a);
+            a = butterfly_sum(a);
             if (lane == 0) nred[wave * MV + j] = a;
         }
         __syncthreads();

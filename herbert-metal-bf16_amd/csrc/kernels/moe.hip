@@ -408,15 +408,16 @@ extern "C" __global__ __launch_bounds__(256) void HB_NAME(const u16* __restrict_
     const u64 base = (u64)r * D;
     float a = 0.0f;
 #pragma unroll
-    for (u32 i = t; i < D; i += 256) a = __builtin_fmaf(bf16_to_f32(xn[base + i]), bf16_to_f32(gate[i]), a);
-#pragma unroll
-    for (int s = 32; s >= 1; s >>= 1) a += __shfl_xor(a, s, 64);
+    for (u32 i = 0; i < D / 256; i++)
+        a = __builtin_fmaf(bf16_to_f32(xn[base + t + 256 * i]), bf16_to_f32(gate[t + 256 * i]), a);
+    a = butterfly_sum(a);
     if (lane == 0) red[t >> 6] = a;
     __syncthreads();
     const float dot = ((red[0] + red[1]) + red[2]) + red[3];
     const float g = round_bf16(hb_sigmoid(round_bf16(dot)));
 #pragma unroll
-    for (u32 i = t; i < D; i += 256) {
+    for (u32 j = 0; j < D / 256; j++) {
+        const u32 i = t + 256 * j;
         const float s = round_bf16(g * bf16_to_f32(sh[base + i]));
         const float o = round_bf16(bf16_to_f32(ex[base + i]) + s);
         x[base + i] = (u16)f32_to_bf16(bf16_to_f32(x[base + i]) + o);
@@ -428,34 +429,69 @@ extern "C" __global__ __launch_bounds__(256) void HB_NAME(const u16* __restrict_
 // (thread t's fma chain over t, t+256, ..., the 64-lane butterfly, the 4
 // waves in order), m = ss * f32(1/D) + eps, inv = 1/sqrt(m) correctly
 // rounded, y = bf16((x * inv) * w) with w + 1 for plus_one -- the same
-// arithmetic as the matvec's fused XSrc::Norm. ----
+// arithmetic as the matvec's fused XSrc::Norm.  The row and the weights come
+// and go in 16-byte chunks, both loaded before the sum (one memory latency);
+// the sum's order reads the row back from LDS. ----
 static_assert(D % 256 == 0, "rmsnorm: d a multiple of 256");
+constexpr u32 CELLS = D / 8, CPT = (CELLS + 255) / 256;  // 16-byte chunks, of a thread
+// A row, the weights and y may start at any element of a buffer.
+typedef u32x4 chunk_t __attribute__((aligned(2)));
 
 extern "C" __global__ __launch_bounds__(256) void HB_NAME(const u16* __restrict__ x,
                                                             const u16* __restrict__ w,
                                                             u16* __restrict__ y, u32 rows) {
     __shared__ float red[4];
+    __shared__ u32x4 row[CELLS];
     const u32 r = blockIdx.x, t = threadIdx.x, lane = t & 63u;
     if (r >= rows) return;
     const u64 base = (u64)r * D;
-    float a = 0.0f;
+    const chunk_t* x4 = (const chunk_t*)(x + base);
+    const chunk_t* w4 = (const chunk_t*)w;
+    u32x4 xv[CPT], wv[CPT];
 #pragma unroll
-    for (u32 i = t; i < D; i += 256) {
-        const float v = bf16_to_f32(x[base + i]);
-        a = __builtin_fmaf(v, v, a);
+    for (u32 i = 0; i < CPT; i++) {
+        const u32 c = t + 256 * i;
+        if (CELLS % 256 == 0 || c < CELLS) xv[i] = x4[c];
     }
 #pragma unroll
-    for (int s = 32; s >= 1; s >>= 1) a += __shfl_xor(a, s, 64);
+    for (u32 i = 0; i < CPT; i++) {
+        const u32 c = t + 256 * i;
+        if (CELLS % 256 == 0 || c < CELLS) wv[i] = w4[c];
+    }
+#pragma unroll
+    for (u32 i = 0; i < CPT; i++) {
+        const u32 c = t + 256 * i;
+        if (CELLS % 256 == 0 || c < CELLS) row[c] = xv[i];
+    }
+    __syncthreads();
+    const u16* xs = (const u16*)row;
+    float a = 0.0f;
+#pragma unroll
+    for (u32 i = 0; i < D / 256; i++) {
+        const float v = bf16_to_f32(xs[t + 256 * i]);
+        a = __builtin_fmaf(v, v, a);
+    }
+    a = butterfly_sum(a);
     if (lane == 0) red[t >> 6] = a;
     __syncthreads();
     const float ss = ((red[0] + red[1]) + red[2]) + red[3];
     const float inv_d = 1.0f / (float)D, eps = __uint_as_float((u32)HB_EPS);
     const float inv = __fdiv_rn(1.0f, __fsqrt_rn(ss * inv_d + eps));
 #pragma unroll
-    for (u32 i = t; i < D; i += 256) {
-        float wf = bf16_to_f32(w[i]);
-        if (HB_PLUS1) wf = wf + 1.0f;
-        y[base + i] = (u16)f32_to_bf16((bf16_to_f32(x[base + i]) * inv) * wf);
+    for (u32 i = 0; i < CPT; i++) {
+        const u32 c = t + 256 * i;
+        if (CELLS % 256 != 0 && c >= CELLS) break;
+        u32x4 o;
+#pragma unroll
+        for (u32 e = 0; e < 4; e++) {
+            float w0 = bf16_lo(wv[i][e]), w1 = bf16_hi(wv[i][e]);
+            if (HB_PLUS1) {
+                w0 = w0 + 1.0f;
+                w1 = w1 + 1.0f;
+            }
+            o[e] = pack_bf16x2((bf16_lo(xv[i][e]) * inv) * w0, (bf16_hi(xv[i][e]) * inv) * w1);
+        }
+        ((chunk_t*)(y + base))[c] = o;
     }
 }
 #endif

@@ -196,6 +196,25 @@ def test_moe_layer_through_picked_kernels(gpu):
     gpu.free(Wdn)
 
 
+@pytest.mark.parametrize("d,rows,at", [(256, 3, 0), (2304, 5, 1), (2560, 2, 7)])
+def test_rmsnorm_any_start(gpu, d, rows, at):
+    """Rows, weights and outputs that start `at` elements into their buffers
+    (2-byte aligned only), one chunk a row of threads and ragged counts."""
+    x = hb.normal_bf16(53, 2.0, (at + rows * d,))
+    w = hb.normal_bf16(54, 0.1, (at + d,))
+    X, Wb, Y = gpu.alloc_with(x), gpu.alloc_with(w), gpu.alloc_with(np.full(at + rows * d + 3, 0x7FC1, np.uint16))
+    try:
+        k = gpu.pipeline(hb.rmsnorm(d, 1e-6, True))
+        gpu.launch(k, [hb.r(X, 2 * at), hb.r(Wb, 2 * at), hb.r(Y, 2 * at)], rows)
+        got = gpu.download(Y, np.uint16, at + rows * d + 3)
+    finally:
+        for b in (X, Wb, Y):
+            gpu.free(b)
+    want = orc.rmsnorm_rows(x[at:].reshape(rows, d), w[at:].copy(), 1e-6, True, 0)
+    assert np.array_equal(got[at:at + rows * d].reshape(rows, d), want)
+    assert np.all(got[:at] == 0x7FC1) and np.all(got[at + rows * d:] == 0x7FC1)
+
+
 def test_rmsnorm_kernel_bit_exact(gpu):
     """The block's input norm: the oracle restates the kernel's summation
     order, so every output bit matches (rows of 2048 and of 2560)."""
