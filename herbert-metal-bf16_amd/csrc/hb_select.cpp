@@ -1266,6 +1266,19 @@ int hb_engine_experts(hb_engine* e, uint32_t experts, uint32_t top_k, uint32_t h
             add_gu("mma_swiglu_wnt", d, false);
         }
         add_gu("mma_swiglu_n256", swi_desc(256), false);
+        if (bm <= 32) {
+            // Few rows per expert (a decode batch, a short prompt): 64-wide
+            // W tiles of 128 K, two or three in flight in each of four or
+            // more workgroups a CU, where 128 x 64 K tiles had one in flight
+            // in two (8 tokens: 52 -> 38 us, 50 tokens: 141 -> 128).
+            for (uint32_t dbuf : {1u, 2u}) {
+                hb_desc d = swi_desc(64, 1, 2);
+                d.bk = 128;
+                d.dbuf = dbuf;
+                d.w_nt = 1;
+                add_gu("mma_swiglu_n64_k128_s" + std::to_string(dbuf + 1) + "_wnt", d, false);
+            }
+        }
         if (bm >= 32) add_gu("mma_swiglu_w2x2", swi_desc(128, 2, 2), false);
         add_dn("mma", gemm_desc(inter, hidden, HB_ROWS_SCATTER, bm, 128));
         add_dn("mma_n256", gemm_desc(inter, hidden, HB_ROWS_SCATTER, bm, 256));
@@ -1279,6 +1292,15 @@ int hb_engine_experts(hb_engine* e, uint32_t experts, uint32_t top_k, uint32_t h
             hb_desc d2 = gemm_desc(inter, hidden, HB_ROWS_SCATTER, bm, 128);
             d2.w_nt = 1;
             add_dn("mma_wnt", d2);
+            if (bm <= 32) {
+                // As above for down's shorter K: four stages of 64 K (8
+                // tokens: 21 -> 19 us, 50 tokens: 67 -> 63).
+                hb_desc d4 = gemm_desc(inter, hidden, HB_ROWS_SCATTER, bm, 64, 1, 4, 3);
+                d4.m_first = d.m_first;
+                d4.w_nt = 1;
+                d4.order = 1;
+                add_dn(d4.m_first ? "mma_n64_s4_mf_wnt" : "mma_n64_s4_nf_wnt", d4);
+            }
             if (bm >= 32) {
                 // 256-wide W tiles, 8 waves, 3 stages, in the same order.
                 hb_desc d3 = gemm_desc(inter, hidden, HB_ROWS_SCATTER, bm, 256, 2, 4, 2);
