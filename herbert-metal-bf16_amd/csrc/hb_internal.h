@@ -59,6 +59,11 @@ struct Kernel {
     // A split-K GEMM (desc.ksplit > 1): the kernel that adds its parts'
     // slabs and applies Out, launched after it by every launch of this one.
     int32_t reduce = -1;
+    // A dense GEMM's choice per row count (hb_engine_gemm, gate_up): a
+    // launch over m rows runs the first (rows, kernel) with m <= rows, and
+    // past the last this kernel itself.  Such an entry shares its kernel's
+    // function, not its module.
+    std::vector<std::pair<uint32_t, int32_t>> by_rows;
 };
 
 // The descriptor kind of a split-K GEMM's second kernel (built by the
@@ -108,6 +113,11 @@ int launch_ptrs(hb_gpu* g, int32_t kernel, void* const* ptrs, const uint64_t* si
                 uint32_t m);
 // The descriptor a kernel was built from (defaults filled), or null.
 const hb_desc* kernel_desc(hb_gpu* g, int32_t kernel);
+// One more entry for kernel `base` that launches the kernels of `by_rows`
+// (ascending rows) on fewer rows; base itself if there are none.
+int32_t with_rows(hb_gpu* g, int32_t base, const std::vector<std::pair<uint32_t, int32_t>>& by_rows);
+// The (rows, kernel) choices of an entry, empty for a plain kernel.
+std::vector<std::pair<uint32_t, int32_t>> rows_of_kernel(hb_gpu* g, int32_t kernel);
 // The device address of the static scratch (hb_static.hip) on `device`,
 // which must be current: looked up, and its state word written, once per
 // device.

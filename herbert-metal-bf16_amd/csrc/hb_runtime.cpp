@@ -255,17 +255,52 @@ static int launch_raw(hb_gpu* g, const Kernel& k, void** ptrs, uint32_t nptr, ui
     return launch_one(g, r, q, 3, m, groups_of(r.desc, m));
 }
 
+// The kernel a launch of entry `kernel` over m rows runs.
+static const Kernel& kernel_for(hb_gpu* g, int32_t kernel, uint32_t m) {
+    const Kernel& k = g->kernels[kernel];
+    for (const auto& v : k.by_rows)
+        if (m <= v.first) return g->kernels[v.second];
+    return k;
+}
+
+// The workspace of any launch of entry `kernel` over up to m rows: of every
+// row range's kernel at its most rows, not only of the one that m takes, so
+// that a first launch at the largest rows sizes it for all.
+static uint64_t workspace_for(hb_gpu* g, int32_t kernel, uint32_t m) {
+    const Kernel& k = g->kernels[kernel];
+    uint64_t most = workspace_of(kernel_for(g, kernel, m).desc, m);
+    for (const auto& v : k.by_rows) {
+        const uint64_t b = workspace_of(g->kernels[v.second].desc, v.first);
+        most = b > most ? b : most;
+    }
+    return most;
+}
+
+int32_t with_rows(hb_gpu* g, int32_t base, const std::vector<std::pair<uint32_t, int32_t>>& by_rows) {
+    if (by_rows.empty()) return base;
+    Kernel k = g->kernels[base];
+    k.module = nullptr;  // unloaded with the kernel it belongs to
+    k.by_rows = by_rows;
+    g->kernels.push_back(k);
+    return (int32_t)(g->kernels.size() - 1);
+}
+
+std::vector<std::pair<uint32_t, int32_t>> rows_of_kernel(hb_gpu* g, int32_t kernel) {
+    if (kernel < 0 || (size_t)kernel >= g->kernels.size()) return {};
+    return g->kernels[kernel].by_rows;
+}
+
 int launch_ptrs(hb_gpu* g, int32_t kernel, void* const* ptrs, const uint64_t* sizes, uint32_t nbind,
                 uint32_t m) {
     if (kernel < 0 || (size_t)kernel >= g->kernels.size())
         return fail(HB_ERR_INVALID, "no kernel " + std::to_string(kernel));
-    const Kernel& k = g->kernels[kernel];
+    const Kernel& k = kernel_for(g, kernel, m);
     if (nbind != k.em.nbind)
         return fail(HB_ERR_INVALID, k.em.name + ": " + std::to_string(nbind) +
                                         " bindings given, it takes " + std::to_string(k.em.nbind));
     int rc = check_bindings(k.desc, sizes, nbind, m);
     if (rc) return fail(rc, k.em.name + ": " + hb_last_error());
-    if ((rc = ensure_ws(g, workspace_of(k.desc, m)))) return rc;
+    if ((rc = ensure_ws(g, workspace_for(g, kernel, m)))) return rc;
     void* p[10];
     for (uint32_t i = 0; i < nbind; i++) p[i] = ptrs[i];
     return launch_raw(g, k, p, nbind, m, groups_of(k.desc, m));
@@ -504,7 +539,7 @@ const char* hb_kernel_name(hb_gpu* g, int32_t kernel) {
 
 uint32_t hb_kernel_groups(hb_gpu* g, int32_t kernel, uint32_t m) {
     if (kernel < 0 || (size_t)kernel >= g->kernels.size()) return 0;
-    return groups_of(g->kernels[kernel].desc, m);
+    return groups_of(kernel_for(g, kernel, m).desc, m);
 }
 
 uint32_t hb_kernel_bindings(hb_gpu* g, int32_t kernel) {
@@ -545,7 +580,7 @@ static int prepare(hb_gpu* g, const hb_op* ops, uint32_t nops, std::vector<Ready
         const hb_op& op = ops[i];
         if (op.kernel < 0 || (size_t)op.kernel >= g->kernels.size())
             return fail(HB_ERR_INVALID, "no kernel " + std::to_string(op.kernel));
-        const Kernel& k = g->kernels[op.kernel];
+        const Kernel& k = kernel_for(g, op.kernel, op.m);
         if (op.nbind != k.em.nbind || op.nbind > 8)
             return fail(HB_ERR_INVALID, k.em.name + ": wrong number of bindings");
         uint64_t sizes[10];
@@ -557,7 +592,7 @@ static int prepare(hb_gpu* g, const hb_op* ops, uint32_t nops, std::vector<Ready
         }
         int rc = check_bindings(k.desc, sizes, op.nbind, op.m);
         if (rc) return fail(rc, k.em.name + ": " + hb_last_error());
-        if ((rc = ensure_ws(g, workspace_of(k.desc, op.m)))) return rc;
+        if ((rc = ensure_ws(g, workspace_for(g, op.kernel, op.m)))) return rc;
         ready[i].k = &k;
         ready[i].n = op.nbind;
         ready[i].m = op.m;

@@ -277,6 +277,15 @@ const Form kMoreForms[] = {
     {"mma_t128x64_s4_w8", 128, 64, 64, 4, 2, 16, 3, 1, 1},
     {"mma_t64x64", 64, 64, 64, 2, 2, 16, 2, 1, 1},
     {"mma_t32x64", 32, 64, 64, 1, 4, 16, 2, 1, 1},
+    // Short prompts (one to four row tiles): column tiles narrow enough to
+    // reach every CU without a split and its second launch, stages as deep
+    // as LDS holds (9216 x 2560 has no such tile: kSplitForms).  57 rows of
+    // 2560 x 18432: 27.6 -> 23.0 us; 200 rows of 4096 x 2560: 18.1 -> 15.2.
+    {"mma_t64x80_k128_s4", 64, 80, 128, 4, 1, 16, 3, 1, 0},
+    {"mma_t64x96_s4", 64, 96, 64, 2, 2, 16, 3, 1, 1},
+    {"mma_t64x64_s4", 64, 64, 64, 4, 1, 16, 3, 1, 1},
+    {"mma_t32x96_k128_s4", 32, 96, 128, 2, 2, 16, 3, 1, 1},
+    {"mma_t128x80_s3", 128, 80, 64, 2, 1, 16, 2, 1, 1},
     // Eight waves in two groups taking turns between memory and MFMA phases
     // (hb_desc.sched 1), four stages of 32 K: 256 x 288 tiles fill exactly
     // two rounds of the CUs on 2048 x 18432 (and 4608: 128 tiles).
@@ -310,6 +319,11 @@ const Form kSplitForms[] = {
     {"mma_t128x192_w8_s4_ks2", 128, 192, 64, 2, 4, 16, 3, 1, 1, 0, 0, 2},
     {"mma_t128x192_w8_s4_ks4", 128, 192, 64, 2, 4, 16, 3, 1, 1, 0, 0, 4},
     {"mma_t128x192_w8_s4_ks8", 128, 192, 64, 2, 4, 16, 3, 1, 1, 0, 0, 8},
+    // Short prompts: 57 rows of 9216 x 2560 20.8 -> 15.2 us.
+    {"mma_t64x96_w8_s4_ks8", 64, 96, 64, 4, 2, 16, 3, 1, 0, 0, 0, 8},
+    {"mma_t32x64_k128_s4_ks3", 32, 64, 128, 1, 4, 16, 3, 1, 1, 0, 0, 3},
+    {"mma_t64x64_k128_s3_ks4", 64, 64, 128, 1, 4, 16, 2, 1, 1, 0, 0, 4},
+    {"mma_t128x48_s4_ks2", 128, 48, 64, 4, 1, 16, 3, 1, 1, 0, 0, 2},
     {"pp_t256x160_k64_ks2", 256, 160, 64, 4, 2, 16, 2, 1, 1, 0, 1, 2},
     {"pp_t256x160_k64_ks4", 256, 160, 64, 4, 2, 16, 2, 1, 1, 0, 1, 4},
     {"pp_t128x160_k64_ks2", 128, 160, 64, 4, 2, 16, 3, 1, 1, 0, 1, 2},
@@ -512,7 +526,7 @@ struct hb_engine {
     // sees, and the ranking of warm runs is not the ranking in the step.
     int pick_flagged(const std::string& what, const std::vector<Cand>& c,
                      const std::vector<bool>& eligible, size_t* best, double* best_s,
-                     bool cold = false) {
+                     bool cold = false, std::vector<double>* medians = nullptr) {
         auto t0 = std::chrono::steady_clock::now();
         if (c.empty() || std::none_of(eligible.begin(), eligible.end(), [](bool e) { return e; }))
             return fail(HB_ERR_INVALID, what + ": no eligible candidate");
@@ -549,6 +563,83 @@ struct hb_engine {
         last_timed = std::chrono::steady_clock::now();
         *best = b;
         if (best_s) *best_s = med[b];
+        if (medians) *medians = med;
+        return HB_OK;
+    }
+
+    // The kernels of a choice made at m rows for launches over fewer: a
+    // bucket's kernel also runs the prompts that end in it, and the tiles
+    // that fill the chip at its full rows often do not below (17408 x 5120
+    // by 256 x 160 tiles: one full round at 2048 rows, and the same 283 us
+    // at 1100, where 128 x 192 tiles take 207).  At 5/8, 3/4 and 7/8 of m (a
+    // bucket's rows begin past its half; a first bucket of 64 rows or less:
+    // 1/4 and 1/2) the six candidates of the least predicted time, the time
+    // at m by the rounds of workgroups the 256 CUs run, are timed against
+    // the kernel of m, and one that is at least 3% faster is kept for
+    // launches of up to those rows.  *kernel becomes an entry that launches
+    // by rows.
+    int pick_rows(const std::string& what, const std::vector<Cand>& c, const std::vector<bool>& eligible,
+                  const std::vector<double>& med, size_t best, hb_range state, uint32_t m, int32_t* kernel) {
+        auto t0 = std::chrono::steady_clock::now();
+        std::vector<uint32_t> at;
+        if (m > 64)
+            at = {(5 * m + 7) / 8, (3 * m + 3) / 4, (7 * m + 7) / 8};
+        else if (m >= 16)
+            at = {(m + 3) / 4, (m + 1) / 2};
+        auto rounds = [&](size_t i, uint32_t rows) {
+            const hb_desc& d = *kernel_desc(g, c[i].kernel);
+            const uint64_t lds = (uint64_t)(d.dbuf + 1) * (d.bm + d.bn) * d.bk * 2;
+            const uint64_t per = d.lds_dma ? std::max<uint64_t>(1, 160 * 1024 / std::max<uint64_t>(lds, 1)) : 4;
+            const uint64_t slots = 256 * std::min<uint64_t>(per, 4);
+            return (double)((groups_of(d, rows) + slots - 1) / slots);
+        };
+        std::vector<std::pair<uint32_t, int32_t>> by_rows;
+        int rc = HB_OK;
+        for (uint32_t rows : at) {
+            std::vector<std::pair<double, size_t>> order;
+            for (size_t i = 0; i < c.size(); i++)
+                if (eligible[i] && i != best) order.push_back({med[i] * rounds(i, rows) / rounds(i, m), i});
+            std::sort(order.begin(), order.end());
+            if (order.size() > 6) order.resize(6);
+            std::vector<size_t> tried = {best};
+            for (const auto& o : order) tried.push_back(o.second);
+            uint32_t st[4] = {0, 0, 0, rows};
+            if ((rc = hb_upload(g, state.buf, state.offset, st, 16))) break;
+            std::vector<std::vector<double>> times(tried.size());
+            uint32_t reps = 1;
+            for (int round = 0; round < 4 && !rc; round++)
+                for (size_t i = 0; i < tried.size() && !rc; i++) {
+                    std::vector<hb_op> ops = c[tried[i]].ops;
+                    for (auto& op : ops) op.m = rows;
+                    double s;
+                    if ((rc = run_ops(ops, reps, true, &s))) break;
+                    if (round == 0) {  // the first run of each warms it
+                        if (i == 0) reps = (uint32_t)std::min(32.0, std::max(2.0, std::ceil(1e-3 / std::max(s, 1e-6))));
+                        continue;
+                    }
+                    times[i].push_back(s / reps);
+                }
+            if (rc) break;
+            size_t b = 0;
+            for (size_t i = 0; i < tried.size(); i++) {
+                std::sort(times[i].begin(), times[i].end());
+                if (times[i][1] < times[b][1]) b = i;
+            }
+            const bool other = b != 0 && times[b][1] < 0.97 * times[0][1];
+            const int32_t k = c[tried[other ? b : 0]].kernel;
+            if (!by_rows.empty() && by_rows.back().second == k)
+                by_rows.back().first = rows;
+            else
+                by_rows.push_back({rows, k});
+            logf("[autotune] %s: %u rows %s %.3f ms, %s %.3f ms", what.c_str(), rows, c[best].name.c_str(),
+                 times[0][1] * 1e3, c[tried[b]].name.c_str(), times[b][1] * 1e3);
+        }
+        uint32_t st[4] = {0, 0, 0, m};
+        const int rc2 = hb_upload(g, state.buf, state.offset, st, 16);
+        if (rc || rc2) return rc ? rc : rc2;
+        while (!by_rows.empty() && by_rows.back().second == c[best].kernel) by_rows.pop_back();
+        *kernel = with_rows(g, c[best].kernel, by_rows);
+        autotune_seconds += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
         return HB_OK;
     }
 
@@ -795,9 +886,13 @@ int hb_engine_gemm(hb_engine* e, uint32_t k, uint32_t n, uint32_t out, hb_range 
     uint32_t row_bytes = n * (out == HB_OUT_F32 ? 4 : 2);
     if ((rc = e->check_candidates(what, c, eligible, state, y, out == HB_OUT_F32, m, row_bytes))) return rc;
     size_t best;
-    if ((rc = e->pick_flagged(what, c, eligible, &best, nullptr, true))) return rc;
-    e->gemm_pick[key] = c[best].kernel;
-    *kernel = c[best].kernel;
+    std::vector<double> med;
+    int32_t kept;
+    if ((rc = e->pick_flagged(what, c, eligible, &best, nullptr, true, &med)) ||
+        (rc = e->pick_rows(what, c, eligible, med, best, state, m, &kept)))
+        return rc;
+    e->gemm_pick[key] = kept;
+    *kernel = kept;
     return HB_OK;
 }
 
@@ -857,8 +952,14 @@ int hb_engine_gate_up(hb_engine* e, uint32_t h, uint32_t inter, hb_range state, 
     if (fswi == 1) return c[0].name == "apart" ? keep(gk, sk) : keep(c[0].kernel, -1);
     if ((rc = e->check_candidates(what, c, eligible, state, hout, false, m, inter * 2))) return rc;
     size_t best;
-    if ((rc = e->pick_flagged(what, c, eligible, &best, nullptr, true))) return rc;
-    return best == 0 ? keep(gk, sk) : keep(c[best].kernel, -1);
+    std::vector<double> med;
+    if ((rc = e->pick_flagged(what, c, eligible, &best, nullptr, true, &med))) return rc;
+    if (best == 0) return keep(gk, sk);
+    // Fewer rows take another fused form (the apart pair binds another Y).
+    eligible[0] = eligible[0] && fswi != 2;
+    int32_t kept;
+    if ((rc = e->pick_rows(what, c, eligible, med, best, state, m, &kept))) return rc;
+    return keep(kept, -1);
 }
 
 int hb_engine_matvec(hb_engine* e, uint32_t k, uint32_t n, uint32_t out, uint32_t mv_m,
@@ -1349,13 +1450,22 @@ static std::string desc_text(hb_gpu* g, int32_t k) {
     return s;
 }
 
+// The choices of a kernel entry by rows, after its own fields: for each the
+// rows, the kernel's name and its descriptor.
+static std::string rows_text(hb_gpu* g, int32_t k) {
+    std::string s;
+    for (const auto& v : rows_of_kernel(g, k)) s += "\t" + std::to_string(v.first) + "\t" + desc_text(g, v.second);
+    return s;
+}
+
 int hb_engine_picks(hb_engine* e, char* buf, uint64_t cap, uint64_t* len) {
     if (!e->g) return fail(HB_ERR_INVALID, "picks: an engine without a context");
     std::string s;
-    for (const auto& kv : e->gemm_pick) s += "gemm\t" + kv.first + "\t" + desc_text(e->g, kv.second) + "\n";
+    for (const auto& kv : e->gemm_pick) s += "gemm\t" + kv.first + "\t" + desc_text(e->g, kv.second) +
+                                           rows_text(e->g, kv.second) + "\n";
     for (const auto& kv : e->gate_up_pick)
         s += "gate_up\t" + kv.first + "\t" + desc_text(e->g, kv.second.first) + "\t" +
-             desc_text(e->g, kv.second.second) + "\n";
+             desc_text(e->g, kv.second.second) + rows_text(e->g, kv.second.first) + "\n";
     for (const auto& kv : e->mv_pick) {
         int32_t k;
         int rc = e->build(kv.second, &k);
@@ -1409,15 +1519,33 @@ int hb_engine_pin(hb_engine* e, const char* text) {
                 return bad("the descriptor builds " + std::string(hb_kernel_name(e->g, *k)) + ", not " + f[at]);
             return HB_OK;
         };
+        // The (rows, kernel) choices from fields f[at] on (none in text of an
+        // engine without them), onto kernel *k.
+        auto rows_at = [&](size_t at, int32_t* k) -> int {
+            std::vector<std::pair<uint32_t, int32_t>> by_rows;
+            for (; at < f.size(); at += 3) {
+                uint32_t rows, last = by_rows.empty() ? 0 : by_rows.back().first;
+                std::string err;
+                int32_t v;
+                if (*k < 0 || !Tune::parse_u32(f[at], &rows, &err) || rows <= last) return bad("rows " + f[at]);
+                if (int r = kernel_at(at + 1, &v)) return r;
+                const hb_desc *a = kernel_desc(e->g, *k), *b = kernel_desc(e->g, v);
+                if (!b || a->kind != b->kind || a->k != b->k || a->n != b->n || a->out != b->out)
+                    return bad(f[at + 1] + " is no kernel of this choice");
+                by_rows.push_back({rows, v});
+            }
+            *k = with_rows(e->g, *k, by_rows);
+            return HB_OK;
+        };
         int rc;
         if (f.size() < 2) return bad("no key");
         if (f[0] == "gemm") {
             int32_t k;
-            if ((rc = kernel_at(2, &k))) return rc;
+            if ((rc = kernel_at(2, &k)) || (rc = rows_at(4, &k))) return rc;
             e->gemm_pick[f[1]] = k;
         } else if (f[0] == "gate_up") {
             int32_t a, b;
-            if ((rc = kernel_at(2, &a)) || (rc = kernel_at(4, &b))) return rc;
+            if ((rc = kernel_at(2, &a)) || (rc = kernel_at(4, &b)) || (rc = rows_at(6, &a))) return rc;
             e->gate_up_pick[f[1]] = {a, b};
         } else if (f[0] == "mv") {
             int32_t k;

@@ -297,7 +297,11 @@ int hb_engine_buckets(hb_engine *engine, uint32_t *out, uint32_t cap, uint32_t *
  * qwen.rs:2497-2545: max|err| <= max|ref|/64 at m and m - m/3 - 3 rows) and
  * the fastest eligible kept (pick_flagged, qwen.rs:2547-2575), cached under
  * "{k}x{n} {Out}, {m} rows".  W, X, Y and the 16-byte state are the buffers
- * timed on (state[3] and Y restored afterwards).  Logs [autotune] lines. */
+ * timed on (state[3] and Y restored afterwards).  Logs [autotune] lines.
+ * A timed choice also times its best candidates at fewer rows (5/8, 3/4 and
+ * 7/8 of m): *kernel launched over m' rows runs the one kept for m', with
+ * the same bindings; its name and kind are those of m.  Its first launch
+ * sizes the split-K workspace for every row count up to m. */
 int hb_engine_gemm(hb_engine *engine, uint32_t k, uint32_t n, uint32_t out, hb_range state,
                    hb_range w, hb_range x, hb_range y, uint32_t m, int32_t *kernel);
 
@@ -419,7 +423,8 @@ int hb_engine_log_summary(hb_engine *engine);
  * separated -- "gemm" / "gate_up" / "mv" / "experts", the choice's key (as
  * the [autotune] lines print it), then each kernel of the choice as its
  * name and its descriptor's fields (decimal, hb_desc order; "-" for none;
- * experts: the tile rows first).  *len = the text's length; up to cap - 1
+ * experts: the tile rows first); after a dense GEMM's kernels, for each
+ * choice at fewer rows those rows, its kernel's name and fields.  *len = the text's length; up to cap - 1
  * bytes and a terminating zero into buf (buf may be null). */
 int hb_engine_picks(hb_engine *engine, char *buf, uint64_t cap, uint64_t *len);
 /* Seeds the engine's choices with text hb_engine_picks wrote (on this or

@@ -324,6 +324,49 @@ def test_prefill_mlp_from_checkpoint_in_blocks(gpu, tmp_path):
         mlp.free()
 
 
+def test_gemm_choice_by_rows(gpu):
+    """A timed choice launched over fewer rows than it was made at (another
+    kernel may run at each of its row ranges): the ranges' edges and one row,
+    against the oracle, rows past the launch's untouched; the choice pinned in
+    another engine prints the same text, and rows out of order or a kernel of
+    another shape are refused."""
+    m, k, n = 128, 1024, 512
+    x, w = hb.normal_bf16(41, 1.0, (m, k)), hb.normal_bf16(42, 0.02, (n, k))
+    st, W, X = gpu.alloc(16), gpu.alloc_with(w), gpu.alloc_with(x)
+    Y = gpu.alloc(m * n * 2)
+    try:
+        with hb.Engine(gpu, "") as a, hb.Engine(gpu, "") as b:
+            gpu.upload(st, np.array([0, 0, 0, m], np.uint32))
+            kern = a.gemm(k, n, 0, hb.r(st), hb.r(W), hb.r(X), hb.r(Y), m)
+            text = a.picks()
+            b.pin(text)
+            assert b.picks() == text
+            f = text.splitlines()[0].split("\t")
+            assert (len(f) - 4) % 3 == 0
+            for bad in ([*f[:4], "96", *f[2:4], "80", *f[2:4]], [*f[:4], "rows", *f[2:4]]):
+                with pytest.raises(hb.HerbertError, match="rows"):
+                    b.pin("\t".join(bad))
+            other = hb.gemm_mma(k, n + 64, 0)
+            name = gpu.kernel_name(gpu.pipeline(other))
+            fields = " ".join(str(getattr(other.replace(bm=128, bn=128, bk=64, wm=2, wn=2, mfma=16), c)) for c in
+                              hb._DESC_FIELDS)
+            with pytest.raises(hb.HerbertError, match="no kernel of this choice"):
+                b.pin("\t".join([*f[:4], "80", name, fields]))
+            pinned = b.gemm(k, n, 0, hb.r(st), hb.r(W), hb.r(X), hb.r(Y), m)
+            want = orc.gemm(x, w)
+            for kk in (kern, pinned):
+                for rows in (1, 79, 80, 81, 96, 97, 112, 113, 128):
+                    gpu.upload(st, np.array([0, 0, 0, rows], np.uint32))
+                    gpu.upload(Y, np.full((m, n), 0x7FC1, np.uint16))
+                    gpu.launch(kk, [hb.r(st), hb.r(W), hb.r(X), hb.r(Y), hb.r(st), hb.r(st)], rows)
+                    got = gpu.download(Y, np.uint16, m * n).reshape(m, n)
+                    check_close(got[:rows], want[:rows], k, abs_products(x[:rows], w), "%d rows" % rows)
+                    assert np.all(got[rows:] == 0x7FC1), rows
+    finally:
+        for buf in (st, W, X, Y):
+            gpu.free(buf)
+
+
 def test_picks_pinned_in_another_engine(gpu):
     """hb_engine_picks / hb_engine_pin: a second engine seeded with the
     first one's choices returns the same kernels without timing them, and a
