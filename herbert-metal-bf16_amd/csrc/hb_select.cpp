@@ -286,6 +286,9 @@ const Form kMoreForms[] = {
     {"mma_t64x64_s4", 64, 64, 64, 4, 1, 16, 3, 1, 1},
     {"mma_t32x96_k128_s4", 32, 96, 128, 2, 2, 16, 3, 1, 1},
     {"mma_t128x80_s3", 128, 80, 64, 2, 1, 16, 2, 1, 1},
+    // Row tiles of 192 for the row counts between those of 128 and 256.
+    {"mma_t192x160_w8_s3", 192, 160, 64, 4, 2, 16, 2, 1, 1},
+    {"pp_t192x160_k64", 192, 160, 64, 4, 2, 16, 2, 1, 1, 0, 1},
     // Eight waves in two groups taking turns between memory and MFMA phases
     // (hb_desc.sched 1), four stages of 32 K: 256 x 288 tiles fill exactly
     // two rounds of the CUs on 2048 x 18432 (and 4608: 128 tiles).
@@ -354,6 +357,8 @@ const Form kFusedForms[] = {
     {"fused256x80_pp", 256, 160, 64, 4, 2, 16, 2, 1, 1, 0, 1},
     {"fused256x80_pp_b4", 256, 160, 64, 4, 2, 16, 2, 1, 1, 4, 1},
     {"fused128x80_pp", 128, 160, 64, 4, 2, 16, 3, 1, 1, 0, 1},
+    {"fused192x80_w8_s3", 192, 160, 64, 4, 2, 16, 2, 1, 1},
+    {"fused192x80_pp", 192, 160, 64, 4, 2, 16, 2, 1, 1, 0, 1},
     {"fused128x96_w8_s4", 128, 192, 64, 2, 4, 16, 3, 1, 0},
     {"fused128x80_s4", 128, 160, 64, 4, 1, 16, 3, 1, 1},
     {"fused128x40_s4", 128, 80, 64, 4, 1, 16, 3, 1, 1},
