@@ -8,6 +8,7 @@
 // QwenEngine::get (src/metal/qwen.rs:1156-1166).
 #include <hip/hiprtc.h>
 
+#include <algorithm>
 #include <chrono>
 #include <cstdio>
 #include <cstdlib>
@@ -255,7 +256,7 @@ static int launch_raw(hb_gpu* g, const Kernel& k, void** ptrs, uint32_t nptr, ui
     return launch_one(g, r, q, 3, m, groups_of(r.desc, m));
 }
 
-// The kernel a launch of entry `kernel` over m rows runs.
+// The kernel of entry `kernel` for a launch over m rows, by rows alone.
 static const Kernel& kernel_for(hb_gpu* g, int32_t kernel, uint32_t m) {
     const Kernel& k = g->kernels[kernel];
     for (const auto& v : k.by_rows)
@@ -263,17 +264,20 @@ static const Kernel& kernel_for(hb_gpu* g, int32_t kernel, uint32_t m) {
     return k;
 }
 
-// The workspace of any launch of entry `kernel` over up to m rows: of every
-// row range's kernel at its most rows, not only of the one that m takes, so
-// that a first launch at the largest rows sizes it for all.
-static uint64_t workspace_for(hb_gpu* g, int32_t kernel, uint32_t m) {
-    const Kernel& k = g->kernels[kernel];
-    uint64_t most = workspace_of(kernel_for(g, kernel, m).desc, m);
-    for (const auto& v : k.by_rows) {
-        const uint64_t b = workspace_of(g->kernels[v.second].desc, v.first);
-        most = b > most ? b : most;
-    }
-    return most;
+// The kernel a launch of entry `kernel` over m rows runs.  An entry with
+// choices by rows first sizes the workspace for all of them (each at its most
+// rows), so that a first launch at any rows does it for the others; where it
+// cannot grow (a recorded graph holds it, or no memory) and the choice for m
+// needs more than there is, the entry's own kernel runs, as it would without
+// the choices.
+static const Kernel& kernel_to_run(hb_gpu* g, int32_t kernel, uint32_t m) {
+    const Kernel& base = g->kernels[kernel];
+    if (base.by_rows.empty()) return base;
+    const Kernel& k = kernel_for(g, kernel, m);
+    uint64_t want = 0;
+    for (const auto& v : base.by_rows) want = std::max(want, workspace_of(g->kernels[v.second].desc, v.first));
+    if (want > g->ws_bytes && !g->graphs_live && ensure_ws(g, want) != HB_OK) (void)hipGetLastError();
+    return workspace_of(k.desc, m) > g->ws_bytes ? base : k;
 }
 
 int32_t with_rows(hb_gpu* g, int32_t base, const std::vector<std::pair<uint32_t, int32_t>>& by_rows) {
@@ -294,13 +298,13 @@ int launch_ptrs(hb_gpu* g, int32_t kernel, void* const* ptrs, const uint64_t* si
                 uint32_t m) {
     if (kernel < 0 || (size_t)kernel >= g->kernels.size())
         return fail(HB_ERR_INVALID, "no kernel " + std::to_string(kernel));
-    const Kernel& k = kernel_for(g, kernel, m);
+    const Kernel& k = kernel_to_run(g, kernel, m);
     if (nbind != k.em.nbind)
         return fail(HB_ERR_INVALID, k.em.name + ": " + std::to_string(nbind) +
                                         " bindings given, it takes " + std::to_string(k.em.nbind));
     int rc = check_bindings(k.desc, sizes, nbind, m);
     if (rc) return fail(rc, k.em.name + ": " + hb_last_error());
-    if ((rc = ensure_ws(g, workspace_for(g, kernel, m)))) return rc;
+    if ((rc = ensure_ws(g, workspace_of(k.desc, m)))) return rc;
     void* p[10];
     for (uint32_t i = 0; i < nbind; i++) p[i] = ptrs[i];
     return launch_raw(g, k, p, nbind, m, groups_of(k.desc, m));
@@ -580,7 +584,7 @@ static int prepare(hb_gpu* g, const hb_op* ops, uint32_t nops, std::vector<Ready
         const hb_op& op = ops[i];
         if (op.kernel < 0 || (size_t)op.kernel >= g->kernels.size())
             return fail(HB_ERR_INVALID, "no kernel " + std::to_string(op.kernel));
-        const Kernel& k = kernel_for(g, op.kernel, op.m);
+        const Kernel& k = kernel_to_run(g, op.kernel, op.m);
         if (op.nbind != k.em.nbind || op.nbind > 8)
             return fail(HB_ERR_INVALID, k.em.name + ": wrong number of bindings");
         uint64_t sizes[10];
@@ -592,7 +596,7 @@ static int prepare(hb_gpu* g, const hb_op* ops, uint32_t nops, std::vector<Ready
         }
         int rc = check_bindings(k.desc, sizes, op.nbind, op.m);
         if (rc) return fail(rc, k.em.name + ": " + hb_last_error());
-        if ((rc = ensure_ws(g, workspace_for(g, op.kernel, op.m)))) return rc;
+        if ((rc = ensure_ws(g, workspace_of(k.desc, op.m)))) return rc;
         ready[i].k = &k;
         ready[i].n = op.nbind;
         ready[i].m = op.m;

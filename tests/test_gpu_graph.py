@@ -62,3 +62,56 @@ def test_graph_replays_equal_stream_launches():
         g.sync()
     finally:
         g.close()
+
+
+def test_choice_by_rows_under_a_graph():
+    """A dense choice whose kernel for few rows splits K: its first launch
+    sizes the workspace for all its rows, so a graph recorded afterwards
+    leaves every row count runnable; while a graph forbids the growth, the
+    choice's own kernel runs those rows."""
+    g = hb.Gpu(0)
+    m, k, n = 256, 768, 640
+    x, w = hb.normal_bf16(0x5EED0310, 1.0, (m, k)), hb.normal_bf16(0x5EED0311, 0.02, (n, k))
+    plain, split = hb.gemm_mma(k, n, 0, **dict(SPLIT, ksplit=0)), hb.gemm_mma(k, n, 0, **SPLIT)
+
+    def text(d):
+        return "%s\t%s" % (g.kernel_name(g.pipeline(d)), " ".join(str(getattr(d, f)) for f in hb._DESC_FIELDS))
+
+    try:
+        st = g.alloc(16)
+        W, X, Y = g.alloc_with(w), g.alloc_with(x), g.alloc(m * n * 2)
+        b = [hb.r(st), hb.r(W), hb.r(X), hb.r(Y), hb.r(st), hb.r(st)]
+
+        def run(kern, rows):
+            g.upload(st, np.array([0, 0, 0, rows], np.uint32))
+            g.zero(Y)
+            g.launch(kern, b, rows)
+            return g.download(Y, np.uint16, rows * n)
+
+        with hb.Engine(g, "") as e:
+            e.pin("gemm\t%dx%d Bf16, %d rows\t%s\t100\t%s\n" % (k, n, m, text(plain), text(split)))
+            kern = e.gemm(k, n, 0, *b[:4], m)
+            kp = g.pipeline(plain)
+            want = run(kp, 100)
+            gr = g.graph([hb.Op(kp, b, m)])
+            try:
+                assert np.array_equal(run(kern, 100), want)  # no workspace yet, none to be had
+            finally:
+                gr.free()
+            whole = run(kp, m)
+            assert np.array_equal(run(kern, m), whole)  # sizes it for 100 rows as well
+            gr = g.graph([hb.Op(kern, b, m)])
+            try:
+                few = run(kern, 100)
+                assert np.array_equal(few, run(g.pipeline(split), 100))
+                assert np.array_equal(run(kern, 101), run(kp, 101))
+                for _ in range(3):
+                    g.upload(st, np.array([0, 0, 0, m], np.uint32))
+                    g.zero(Y)
+                    gr.launch(1)
+                    g.sync()
+                    assert np.array_equal(g.download(Y, np.uint16, m * n), whole)
+            finally:
+                gr.free()
+    finally:
+        g.close()
