@@ -188,16 +188,48 @@ extern "C" __global__ __launch_bounds__(NT) void HB_NAME(const u16* __restrict__
     // chain over elements t, t+256, ..., the 64 lanes' butterfly, then the 4
     // waves' sums in wave order; m = ss * (1/K) + eps; inv = 1/sqrt(m)
     // (correctly rounded); x' = bf16((x * inv) * w) with w + 1 for plus_one.
+    // The rows and the weights come in 16-byte chunks (CPT a thread and row),
+    // issued by prologue_loads before anything else where they fit in
+    // registers: behind the W stream's loads they would come back after them.
+    // The sum reads the row back from LDS in its own order, and each chunk is
+    // normed in place.
     static_assert(K % 256 == 0, "XSrc::Norm: K a multiple of 256");
     __shared__ float nred[WAVES * MV];
+    constexpr u32 CELLS = K / 8, CPT = (CELLS + 255) / 256;
+    constexpr bool EARLY = MV * CPT + CPT <= 12;  // chunks held: 48 registers
+    typedef u32x4 chunk_t __attribute__((aligned(2)));  // x and wn may start at any element
+    u32x4 xc[EARLY ? MV * CPT : 1], wc[EARLY ? CPT : 1];
+    auto x_chunk = [&](u32 j, u32 c) HB_INLINE2 -> u32x4 {
+        return *((const chunk_t*)(x + (u64)(j < m ? j : m - 1) * K) + c);
+    };
+    auto prologue_loads = [&]() HB_INLINE2 {
+        if constexpr (EARLY) {
+#pragma unroll
+            for (u32 i = 0; i < CPT; i++) {
+                const u32 c = tid + 256 * i;
+                if (CELLS % 256 != 0 && c >= CELLS) break;
+#pragma unroll
+                for (u32 j = 0; j < MV; j++) xc[j * CPT + i] = x_chunk(j, c);
+                wc[i] = *((const chunk_t*)wn + c);
+            }
+        }
+    };
     auto prologue = [&]() HB_INLINE2 {
-        constexpr u32 PER = K / 256;
+#pragma unroll
+        for (u32 i = 0; i < CPT; i++) {
+            const u32 c = tid + 256 * i;
+            if (CELLS % 256 != 0 && c >= CELLS) break;
+#pragma unroll
+            for (u32 j = 0; j < MV; j++) xn4[j * XST + c] = EARLY ? xc[EARLY ? j * CPT + i : 0] : x_chunk(j, c);
+        }
+        __syncthreads();
+        const u16* const xs = (const u16*)xn4;
 #pragma unroll
         for (u32 j = 0; j < MV; j++) {
-            const u32 jj = j < m ? j : m - 1;
             float a = 0.0f;
-            for (u32 i = 0; i < PER; i++) {
-                const float v = bf16_to_f32(x[(u64)jj * K + tid + i * 256]);
+#pragma unroll 10
+            for (u32 i = 0; i < K / 256; i++) {
+                const float v = bf16_to_f32(xs[j * K + tid + i * 256]);
                 a = __builtin_fmaf(v, v, a);
             }
             a = butterfly_sum(a);
@@ -205,20 +237,38 @@ extern "C" __global__ __launch_bounds__(NT) void HB_NAME(const u16* __restrict__
         }
         __syncthreads();
         const float inv_d = 1.0f / (float)K, eps = __uint_as_float((u32)HB_EPS);
-        u16* xn = (u16*)xn4;
+        float inv[MV];
 #pragma unroll
         for (u32 j = 0; j < MV; j++) {
-            const u32 jj = j < m ? j : m - 1;
             float ss = nred[j];
 #pragma unroll
             for (u32 w = 1; w < WAVES; w++) ss = ss + nred[w * MV + j];
             const float mm = ss * inv_d + eps;  // -ffp-contract=off: a mul, then an add
-            const float inv = __fdiv_rn(1.0f, __fsqrt_rn(mm));
-            for (u32 i = 0; i < PER; i++) {
-                const u32 c = tid + i * 256;
-                float wf = bf16_to_f32(wn[c]);
-                if (HB_PLUS1) wf = wf + 1.0f;
-                xn[j * K + c] = (u16)f32_to_bf16((bf16_to_f32(x[(u64)jj * K + c]) * inv) * wf);
+            inv[j] = __fdiv_rn(1.0f, __fsqrt_rn(mm));
+        }
+#pragma unroll
+        for (u32 i = 0; i < CPT; i++) {
+            const u32 c = tid + 256 * i;
+            if (CELLS % 256 != 0 && c >= CELLS) break;
+            const u32x4 wv = EARLY ? wc[EARLY ? i : 0] : (u32x4)*((const chunk_t*)wn + c);
+            float wf[8];
+#pragma unroll
+            for (u32 e = 0; e < 4; e++) {
+                wf[2 * e] = bf16_lo(wv[e]);
+                wf[2 * e + 1] = bf16_hi(wv[e]);
+                if (HB_PLUS1) {
+                    wf[2 * e] = wf[2 * e] + 1.0f;
+                    wf[2 * e + 1] = wf[2 * e + 1] + 1.0f;
+                }
+            }
+#pragma unroll
+            for (u32 j = 0; j < MV; j++) {
+                const u32x4 v = xn4[j * XST + c];
+                u32x4 r;
+#pragma unroll
+                for (u32 e = 0; e < 4; e++)
+                    r[e] = pack_bf16x2((bf16_lo(v[e]) * inv[j]) * wf[2 * e], (bf16_hi(v[e]) * inv[j]) * wf[2 * e + 1]);
+                xn4[j * XST + c] = r;
             }
         }
         __syncthreads();
@@ -256,6 +306,9 @@ extern "C" __global__ __launch_bounds__(NT) void HB_NAME(const u16* __restrict__
     constexpr bool HOIST = HB_XSRC == 2 && HB_PERSIST == 0;
     bool pending = HB_XIN_LDS && !HB_MMA && HOIST;
     (void)pending;
+#if HB_XSRC == 2
+    prologue_loads();
+#endif
 #if HB_XIN_LDS
     if constexpr (!HOIST) prologue();
 #endif

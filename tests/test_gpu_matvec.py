@@ -391,3 +391,30 @@ def test_matvec_mf4_lm_head(gpu, m):
     w = hb.normal_bf16(0x5EED0006, 0.02, (n, k))
     got = run_mv(gpu, x, w, 0, mv_m=m, form=4, split=4, waves=8, persist=1024)
     check_close(got, orc.gemm(x, w), k, abs_products(x, w), "lm_head mf4 m=%d" % m)
+
+
+@pytest.mark.parametrize("m,k,persist", [(1, 256, 0), (1, 2560, 0), (4, 2304, 0), (3, 2560, 4), (2, 9216, 0)])
+def test_norm_prologue_any_start(gpu, m, k, persist):
+    """XSrc::Norm with x and the norm weights one element into their buffers
+    (2-byte aligned), one to 36 chunks a row of threads, held in registers or
+    read again: the bits of the same rows at the buffers' start."""
+    n = 72
+    x, nw = hb.normal_bf16(71, 2.0, (m, k)), hb.normal_bf16(72, 0.1, (k,))
+    w = hb.normal_bf16(73, 0.02, (n, k))
+    pad = np.zeros(1, np.uint16)
+    kern = gpu.pipeline(hb.matvec(k, n, 0, mv_m=m, rows=2, split=1, persist=persist, form=0, xsrc=hb.XSrc.Norm,
+                                  eps=1e-6, plus_one=True))
+    got = []
+    for at in (0, 1):
+        X = gpu.alloc_with(np.concatenate([pad[:at], x.reshape(-1)]))
+        NW = gpu.alloc_with(np.concatenate([pad[:at], nw]))
+        W, Y = gpu.alloc_with(w), gpu.alloc(m * n * 2)
+        try:
+            gpu.launch(kern, [hb.r(W), hb.r(X, 2 * at), hb.r(Y), hb.r(NW, 2 * at)], m)
+            got.append(gpu.download(Y, np.uint16, m * n).reshape(m, n))
+        finally:
+            for b in (X, NW, W, Y):
+                gpu.free(b)
+    assert np.array_equal(got[0], got[1])
+    xn = orc.rmsnorm_rows(x, nw, 1e-6, True, 0)
+    check_close(got[0], orc.gemm(xn, w), k, abs_products(xn, w), "norm prologue")
