@@ -34,10 +34,10 @@ HB_DEV u32 pack_bf16x2(float lo, float hi) { return __builtin_bit_cast(u32, bf16
 HB_DEV float round_bf16(float f) { return bf16_to_f32(__builtin_bit_cast(u16, (__bf16)f)); }
 
 // exp of f32: Cody-Waite reduction by ln 2 and the minimax polynomial of
-// Moshier's Cephes expf, every step an explicit fma, so that the CPU checker
+// Moshier's Cephes expf, every step an explicit fma, so that the CPU oracle
 // built with the same steps gives the same bits.  The scaling by 2^n is one
 // v_ldexp_f32 (one rounding, as the two exact-then-rounded multiplies that the
-// checker does: equal on all 2^32 inputs) and the range ends are selects.
+// oracle does: equal on all 2^32 inputs) and the range ends are selects.
 HB_DEV float exp_core(float x) {
     float n = __builtin_floorf(__builtin_fmaf(x, 1.44269504088896341f, 0.5f));
     float r = __builtin_fmaf(n, -0.693359375f, x);
