@@ -212,7 +212,9 @@ static int load_kernel(hb_gpu* g, const hb_desc& d, Kernel* k) {
 }
 
 // The context's workspace grown to `bytes` (the stream drained first: a
-// launch in flight may still read the old one).
+// launch in flight may still read the old one).  The old one is given back
+// once the new one is there, or before, where only its place makes the room;
+// a growth that fails leaves a workspace of the old size.
 static int ensure_ws(hb_gpu* g, uint64_t bytes) {
     if (bytes <= g->ws_bytes) return HB_OK;
     if (g->graphs_live)
@@ -220,11 +222,23 @@ static int ensure_ws(hb_gpu* g, uint64_t bytes) {
                                     "address (free the graphs first, or record after the largest launch)");
     HB_HIP(hipSetDevice(g->device));
     HB_HIP(hipStreamSynchronize(g->stream));
-    if (g->ws) HB_HIP(hipFree(g->ws));
-    g->ws = nullptr;
-    g->ws_bytes = 0;
     const uint64_t sz = (bytes + (1ull << 20) - 1) & ~((1ull << 20) - 1);
-    HB_HIP(hipMalloc(&g->ws, sz));
+    void* grown = nullptr;
+    hipError_t he = hipMalloc(&grown, sz);
+    if (g->ws && (he == hipSuccess || he == hipErrorOutOfMemory)) {
+        HB_HIP(hipFree(g->ws));
+        g->ws = nullptr;
+        const uint64_t old = g->ws_bytes;
+        g->ws_bytes = 0;
+        if (he != hipSuccess && (he = hipMalloc(&grown, sz)) != hipSuccess &&
+            hipMalloc(&g->ws, old) == hipSuccess)
+            g->ws_bytes = old;
+    }
+    if (he != hipSuccess) {
+        (void)hipGetLastError();  // reported here, not by the next launch
+        return hip_fail(he, "split-K workspace");
+    }
+    g->ws = grown;
     g->ws_bytes = sz;
     return HB_OK;
 }

@@ -1,0 +1,79 @@
+"""The split-K workspace of a context (csrc/hb_runtime.cpp) where memory runs
+out, on a HIP runtime over host memory: what the host allocates and which
+kernels it launches with which pointers."""
+import numpy as np
+import pytest
+
+import host_gpu
+
+SPLIT = dict(bm=128, bn=128, bk=64, wm=2, wn=2, mfma=16, dbuf=1, lds_dma=1, order=1, ksplit=2)
+NONE = 2**64 - 1
+M, K, N = 512, 768, 8192   # a split kernel's slabs over M rows: 32 MiB
+MB = 1 << 20
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    mp = pytest.MonkeyPatch()
+    mp.setenv("HB_CACHE_DIR", "")
+    yield host_gpu.load(tmp_path_factory.mktemp("host"))
+    mp.undo()
+
+
+class Rig:
+    """A context with the operands of an M x K x N GEMM."""
+
+    def __init__(self, hb):
+        self.hb, self.lib = hb, hb.lib
+        hb.lib.fake_limit(NONE)
+        self.g = hb.Gpu(0)
+        g = self.g
+        self.st = g.alloc_with(np.array([0, 0, 0, M], np.uint32))
+        self.bind = [hb.r(b) for b in (self.st, g.alloc(N * K * 2), g.alloc(M * K * 2), g.alloc(M * N * 2), self.st, self.st)]
+        self.split, self.plain = hb.gemm_mma(K, N, 0, **SPLIT), hb.gemm_mma(K, N, 0, **dict(SPLIT, ksplit=0))
+        self.ks, self.kp = g.pipeline(self.split), g.pipeline(self.plain)
+        self.slab = N * 4 * 2  # bytes of both parts' slabs, a row
+
+    def room(self, bytes_):
+        """Memory for `bytes_` more."""
+        self.lib.fake_limit(self.lib.fake_in_use() + bytes_)
+
+    def launches(self, rows, kern):
+        self.lib.fake_forget()
+        self.g.launch(kern, self.bind, rows)
+        return self.last()
+
+    def last(self):
+        return [self.lib.fake_launch_name(i).decode() for i in range(self.lib.fake_launches())]
+
+    def slabs(self, i=0):
+        """Bytes from launch i's slab pointer to the end of its allocation."""
+        return self.lib.fake_launch_span(i, 3)
+
+
+@pytest.fixture()
+def rig(host):
+    r = Rig(host)
+    yield r
+    r.lib.fake_limit(NONE)
+    r.g.close()
+
+
+def test_failed_growth_keeps_the_workspace(rig):
+    """A launch whose slabs find no memory is refused; the workspace of
+    earlier launches stays, and they run as before without allocating."""
+    rig.launches(128, rig.ks)
+    held = rig.lib.fake_in_use()
+    rig.room(4 * MB)
+    with pytest.raises(rig.hb.HerbertError, match="out of memory"):
+        rig.g.launch(rig.ks, rig.bind, M)
+    assert rig.lib.fake_in_use() == held
+    rig.room(0)
+    assert len(rig.launches(128, rig.ks)) == 2 and rig.slabs() >= 128 * rig.slab
+
+
+def test_growth_that_fits_in_the_old_ones_place(rig):
+    """Memory for the new workspace only once the old one is given back."""
+    rig.launches(256, rig.ks)
+    rig.room(M * rig.slab - 256 * rig.slab)
+    assert len(rig.launches(M, rig.ks)) == 2 and rig.slabs() >= M * rig.slab
