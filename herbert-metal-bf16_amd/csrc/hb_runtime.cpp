@@ -616,6 +616,10 @@ static int prepare(hb_gpu* g, const hb_op* ops, uint32_t nops, std::vector<Ready
         ready[i].m = op.m;
         ready[i].groups = groups_of(k.desc, op.m);
     }
+    // A later op's growth may have failed and taken the workspace with it.
+    for (const Ready& x : ready)
+        if (workspace_of(x.k->desc, x.m) > g->ws_bytes)
+            return fail(HB_ERR_HIP, x.k->em.name + ": no memory for the sequence's split-K workspace");
     return HB_OK;
 }
 }  // namespace hb

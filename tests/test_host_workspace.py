@@ -77,3 +77,44 @@ def test_growth_that_fits_in_the_old_ones_place(rig):
     rig.launches(256, rig.ks)
     rig.room(M * rig.slab - 256 * rig.slab)
     assert len(rig.launches(M, rig.ks)) == 2 and rig.slabs() >= M * rig.slab
+
+
+def text(rig, d):
+    return "%s\t%s" % (rig.g.kernel_name(rig.g.pipeline(d)), " ".join(str(getattr(d, f)) for f in rig.hb._DESC_FIELDS))
+
+
+def choice(rig, base, *by_rows, rows=M):
+    """The handle of a pinned choice: `base`, and (rows, desc) below it."""
+    line = "gemm\t%dx%d Bf16, %d rows\t%s" % (K, N, rows, text(rig, base))
+    for at, d in by_rows:
+        line += "\t%d\t%s" % (at, text(rig, d))
+    with rig.hb.Engine(rig.g, "") as e:
+        e.pin(line + "\n")
+        return e.gemm(K, N, 0, *rig.bind[:4], rows)
+
+
+def test_sequence_whose_later_op_finds_no_memory(rig):
+    """A split kernel, then a choice whose growth fails: the choice falls back
+    to its own kernel and the first op keeps slabs of the size it needs."""
+    kern = choice(rig, rig.plain, (300, rig.split))
+    ops = [rig.hb.Op(rig.ks, rig.bind, 128), rig.hb.Op(kern, rig.bind, 300)]
+    rig.launches(128, rig.ks)
+    rig.room(0)
+    rig.lib.fake_forget()
+    rig.g.time_ops(ops, 1)
+    assert rig.last() == [rig.g.kernel_name(rig.ks), "gemm_splitk_%d_bf16_s2" % N, rig.g.kernel_name(rig.kp)]
+    assert rig.slabs() >= 128 * rig.slab
+
+
+@pytest.mark.parametrize("entry", ["time_ops", "graph"])
+def test_sequence_that_lost_the_workspace_is_refused(rig, entry):
+    """Where the growth for a later op leaves no workspace at all, the whole
+    sequence is refused before anything is launched."""
+    kern = choice(rig, rig.plain, (300, rig.split))
+    ops = [rig.hb.Op(rig.ks, rig.bind, 128), rig.hb.Op(kern, rig.bind, 300)]
+    rig.launches(128, rig.ks)
+    rig.lib.fake_forget()
+    rig.lib.fake_limit(0)
+    with pytest.raises(rig.hb.HerbertError, match="workspace"):
+        getattr(rig.g, entry)(ops)
+    assert rig.last() == []
