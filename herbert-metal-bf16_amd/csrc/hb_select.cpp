@@ -1491,6 +1491,17 @@ int hb_engine_picks(hb_engine* e, char* buf, uint64_t cap, uint64_t* len) {
     return HB_OK;
 }
 
+// The rows of a dense choice's key ("..., 128 rows"); 0 if it names none.
+static uint32_t key_rows(const std::string& key) {
+    const size_t at = key.rfind(", "), end = key.rfind(" rows");
+    uint32_t m;
+    std::string err;
+    if (at == std::string::npos || end == std::string::npos || end < at + 2 || end + 5 != key.size() ||
+        !Tune::parse_u32(key.substr(at + 2, end - at - 2), &m, &err))
+        return 0;
+    return m;
+}
+
 int hb_engine_pin(hb_engine* e, const char* text) {
     if (!e->g) return fail(HB_ERR_INVALID, "pin: an engine without a context");
     std::istringstream in(text ? text : "");
@@ -1525,14 +1536,17 @@ int hb_engine_pin(hb_engine* e, const char* text) {
             return HB_OK;
         };
         // The (rows, kernel) choices from fields f[at] on (none in text of an
-        // engine without them), onto kernel *k.
+        // engine without them), onto kernel *k: rows ascending, up to those
+        // of the key, which the split-K workspace is sized for.
         auto rows_at = [&](size_t at, int32_t* k) -> int {
             std::vector<std::pair<uint32_t, int32_t>> by_rows;
+            const uint32_t most = key_rows(f[1]);
             for (; at < f.size(); at += 3) {
                 uint32_t rows, last = by_rows.empty() ? 0 : by_rows.back().first;
                 std::string err;
                 int32_t v;
-                if (*k < 0 || !Tune::parse_u32(f[at], &rows, &err) || rows <= last) return bad("rows " + f[at]);
+                if (*k < 0 || !Tune::parse_u32(f[at], &rows, &err) || rows <= last || rows > most)
+                    return bad("rows " + f[at]);
                 if (int r = kernel_at(at + 1, &v)) return r;
                 const hb_desc *a = kernel_desc(e->g, *k), *b = kernel_desc(e->g, v);
                 if (!b || a->kind != b->kind || a->k != b->k || a->n != b->n || a->out != b->out)

@@ -1,0 +1,53 @@
+"""hb_engine_pin / hb_engine_picks (csrc/hb_select.cpp) over a HIP runtime on
+host memory: which text a choice by rows may be read from."""
+import numpy as np
+import pytest
+
+import host_gpu
+
+TILE = dict(bm=128, bn=128, bk=64, wm=2, wn=2, mfma=16, dbuf=1, lds_dma=1, order=1)
+M, K, N = 128, 1024, 512
+
+
+@pytest.fixture(scope="module")
+def hb(tmp_path_factory):
+    mp = pytest.MonkeyPatch()
+    mp.setenv("HB_CACHE_DIR", "")
+    yield host_gpu.load(tmp_path_factory.mktemp("host"))
+    mp.undo()
+
+
+@pytest.fixture()
+def g(hb):
+    g = hb.Gpu(0)
+    yield g
+    g.close()
+
+
+def text(hb, g, d):
+    return "%s\t%s" % (g.kernel_name(g.pipeline(d)), " ".join(str(getattr(d, f)) for f in hb._DESC_FIELDS))
+
+
+def gemm_line(hb, g, base, *by_rows, key="%dx%d Bf16, %d rows" % (K, N, M)):
+    line = "gemm\t%s\t%s" % (key, text(hb, g, base))
+    for rows, d in by_rows:
+        line += "\t%s\t%s" % (rows, text(hb, g, d))
+    return line + "\n"
+
+
+@pytest.mark.parametrize("key,rows,ok", [("%dx%d Bf16, 128 rows" % (K, N), 128, True),
+                                         ("%dx%d Bf16, 128 rows" % (K, N), 129, False),
+                                         ("%dx%d Bf16, 128 rows" % (K, N), 4294967295, False),
+                                         ("%dx%d Bf16" % (K, N), 96, False)])
+def test_rows_within_the_choices_own(hb, g, key, rows, ok):
+    """A range past the rows the choice was made at (they size the split-K
+    workspace), or a choice that names none, is refused."""
+    split = hb.gemm_mma(K, N, 0, **dict(TILE, ksplit=2))
+    line = gemm_line(hb, g, hb.gemm_mma(K, N, 0, **TILE), (rows, split), key=key)
+    with hb.Engine(g, "") as e:
+        if ok:
+            e.pin(line)
+            assert "\t%d\t" % rows in e.picks()
+        else:
+            with pytest.raises(hb.HerbertError, match="rows %d" % rows):
+                e.pin(line)
