@@ -62,8 +62,9 @@ struct Kernel {
     // A dense GEMM's choice per row count (hb_engine_gemm, gate_up): a
     // launch over m rows runs the first (rows, kernel) with m <= rows, and
     // past the last this kernel itself.  Such an entry shares its kernel's
-    // function, not its module.
+    // function, not its module; `rows` is what the choice was made at.
     std::vector<std::pair<uint32_t, int32_t>> by_rows;
+    uint32_t rows = 0;
 };
 
 // The descriptor kind of a split-K GEMM's second kernel (built by the
@@ -113,9 +114,11 @@ int launch_ptrs(hb_gpu* g, int32_t kernel, void* const* ptrs, const uint64_t* si
                 uint32_t m);
 // The descriptor a kernel was built from (defaults filled), or null.
 const hb_desc* kernel_desc(hb_gpu* g, int32_t kernel);
-// One more entry for kernel `base` that launches the kernels of `by_rows`
-// (ascending rows) on fewer rows; base itself if there are none.
-int32_t with_rows(hb_gpu* g, int32_t base, const std::vector<std::pair<uint32_t, int32_t>>& by_rows);
+// One more entry for kernel `base`, chosen at `rows`, that launches the
+// kernels of `by_rows` (ascending rows) on fewer; base itself if there are
+// none.
+int32_t with_rows(hb_gpu* g, int32_t base, const std::vector<std::pair<uint32_t, int32_t>>& by_rows,
+                  uint32_t rows);
 // The (rows, kernel) choices of an entry, empty for a plain kernel.
 std::vector<std::pair<uint32_t, int32_t>> rows_of_kernel(hb_gpu* g, int32_t kernel);
 // The device address of the static scratch (hb_static.hip) on `device`,

@@ -280,25 +280,27 @@ static const Kernel& kernel_for(hb_gpu* g, int32_t kernel, uint32_t m) {
 
 // The kernel a launch of entry `kernel` over m rows runs.  An entry with
 // choices by rows first sizes the workspace for all of them (each at its most
-// rows), so that a first launch at any rows does it for the others; where it
-// cannot grow (a recorded graph holds it, or no memory) and the choice for m
-// needs more than there is, the entry's own kernel runs, as it would without
-// the choices.
+// rows) and for its own kernel at the rows the choice was made at, so that a
+// first launch at any rows does it for the others; where it cannot grow (a
+// recorded graph holds it, or no memory) and the choice for m needs more than
+// there is, the entry's own kernel runs, as it would without the choices.
 static const Kernel& kernel_to_run(hb_gpu* g, int32_t kernel, uint32_t m) {
     const Kernel& base = g->kernels[kernel];
     if (base.by_rows.empty()) return base;
     const Kernel& k = kernel_for(g, kernel, m);
-    uint64_t want = 0;
+    uint64_t want = workspace_of(base.desc, base.rows);
     for (const auto& v : base.by_rows) want = std::max(want, workspace_of(g->kernels[v.second].desc, v.first));
     if (want > g->ws_bytes && !g->graphs_live && ensure_ws(g, want) != HB_OK) (void)hipGetLastError();
     return workspace_of(k.desc, m) > g->ws_bytes ? base : k;
 }
 
-int32_t with_rows(hb_gpu* g, int32_t base, const std::vector<std::pair<uint32_t, int32_t>>& by_rows) {
+int32_t with_rows(hb_gpu* g, int32_t base, const std::vector<std::pair<uint32_t, int32_t>>& by_rows,
+                  uint32_t rows) {
     if (by_rows.empty()) return base;
     Kernel k = g->kernels[base];
     k.module = nullptr;  // unloaded with the kernel it belongs to
     k.by_rows = by_rows;
+    k.rows = rows;
     g->kernels.push_back(k);
     return (int32_t)(g->kernels.size() - 1);
 }

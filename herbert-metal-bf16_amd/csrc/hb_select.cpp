@@ -643,7 +643,7 @@ struct hb_engine {
         const int rc2 = hb_upload(g, state.buf, state.offset, st, 16);
         if (rc || rc2) return rc ? rc : rc2;
         while (!by_rows.empty() && by_rows.back().second == c[best].kernel) by_rows.pop_back();
-        *kernel = with_rows(g, c[best].kernel, by_rows);
+        *kernel = with_rows(g, c[best].kernel, by_rows, m);
         autotune_seconds += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
         return HB_OK;
     }
@@ -1553,7 +1553,7 @@ int hb_engine_pin(hb_engine* e, const char* text) {
                     return bad(f[at + 1] + " is no kernel of this choice");
                 by_rows.push_back({rows, v});
             }
-            *k = with_rows(e->g, *k, by_rows);
+            *k = with_rows(e->g, *k, by_rows, most);
             return HB_OK;
         };
         int rc;

@@ -118,3 +118,21 @@ def test_sequence_that_lost_the_workspace_is_refused(rig, entry):
     with pytest.raises(rig.hb.HerbertError, match="workspace"):
         getattr(rig.g, entry)(ops)
     assert rig.last() == []
+
+
+@pytest.mark.parametrize("swap", [False, True])
+def test_first_launch_sizes_every_row_count(rig, swap):
+    """Whichever of a choice's kernels splits K, its own or that of fewer
+    rows: after a first launch at few rows and a graph, every row count up to
+    the choice's runs the kernel chosen for it."""
+    base, few = (rig.split, rig.plain) if swap else (rig.plain, rig.split)
+    kern = choice(rig, base, (300, few))
+    rig.launches(10, kern)
+    gr = rig.g.graph([rig.hb.Op(rig.kp, rig.bind, M)])
+    try:
+        for rows, d in ((10, few), (300, few), (301, base), (M, base)):
+            assert rig.launches(rows, kern)[0] == rig.g.kernel_name(rig.g.pipeline(d)), rows
+            if d is rig.split:
+                assert rig.slabs() >= rows * rig.slab
+    finally:
+        gr.free()
