@@ -100,6 +100,9 @@ struct hb_gpu {
     // grown before a launch that needs more, freed at hb_close.
     void* ws = nullptr;
     uint64_t ws_bytes = 0;
+    // The smallest size that a choice by rows could not grow it to (no
+    // memory); none after a buffer is freed.
+    uint64_t ws_refused = ~0ull;
     // Recorded graphs alive on this context: they hold the workspace's
     // address, so it may not be reallocated meanwhile.
     int graphs_live = 0;

@@ -283,14 +283,16 @@ static const Kernel& kernel_for(hb_gpu* g, int32_t kernel, uint32_t m) {
 // rows) and for its own kernel at the rows the choice was made at, so that a
 // first launch at any rows does it for the others; where it cannot grow (a
 // recorded graph holds it, or no memory) and the choice for m needs more than
-// there is, the entry's own kernel runs, as it would without the choices.
+// there is, the entry's own kernel runs, as it would without the choices.  A
+// size that found no memory is asked for again once a buffer is freed.
 static const Kernel& kernel_to_run(hb_gpu* g, int32_t kernel, uint32_t m) {
     const Kernel& base = g->kernels[kernel];
     if (base.by_rows.empty()) return base;
     const Kernel& k = kernel_for(g, kernel, m);
     uint64_t want = workspace_of(base.desc, base.rows);
     for (const auto& v : base.by_rows) want = std::max(want, workspace_of(g->kernels[v.second].desc, v.first));
-    if (want > g->ws_bytes && !g->graphs_live && ensure_ws(g, want) != HB_OK) (void)hipGetLastError();
+    if (want > g->ws_bytes && want < g->ws_refused && !g->graphs_live && ensure_ws(g, want) != HB_OK)
+        g->ws_refused = want;  // a drain, a free and failing allocations: not at every launch
     return workspace_of(k.desc, m) > g->ws_bytes ? base : k;
 }
 
@@ -433,6 +435,7 @@ int hb_free(hb_gpu* g, hb_buf buf) {
     HB_HIP(hipFree(g->bufs[buf].ptr));
     g->bufs[buf].live = false;
     g->bufs[buf].ptr = nullptr;
+    g->ws_refused = ~0ull;
     return HB_OK;
 }
 

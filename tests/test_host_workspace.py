@@ -136,3 +136,19 @@ def test_first_launch_sizes_every_row_count(rig, swap):
                 assert rig.slabs() >= rows * rig.slab
     finally:
         gr.free()
+
+
+def test_refused_growth_is_not_tried_at_every_launch(rig):
+    """A choice whose growth found no memory runs its own kernel without
+    asking again, until memory is given back."""
+    kern = choice(rig, rig.plain, (300, rig.split))
+    spare = rig.g.alloc(32 * MB)
+    rig.room(4 * MB)
+    assert rig.launches(300, kern) == [rig.g.kernel_name(rig.kp)]
+    tries = rig.lib.fake_malloc_tries()
+    for _ in range(3):
+        assert rig.launches(300, kern) == [rig.g.kernel_name(rig.kp)]
+    rig.g.time_ops([rig.hb.Op(kern, rig.bind, 300)], 2)
+    assert rig.lib.fake_malloc_tries() == tries
+    rig.g.free(spare)
+    assert rig.launches(300, kern)[0] == rig.g.kernel_name(rig.ks) and rig.slabs() >= 300 * rig.slab
