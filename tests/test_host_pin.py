@@ -51,3 +51,28 @@ def test_rows_within_the_choices_own(hb, g, key, rows, ok):
         else:
             with pytest.raises(hb.HerbertError, match="rows %d" % rows):
                 e.pin(line)
+
+
+def swiglu_line(hb, g, base, *by_rows):
+    line = "gate_up\t%dx%d, %d rows\t%s\t-\t-" % (K, 2 * N, M, text(hb, g, base))
+    for rows, d in by_rows:
+        line += "\t%d\t%s" % (rows, text(hb, g, d))
+    return line + "\n"
+
+
+def test_text_of_every_dense_kind_reads_back(hb, g):
+    """A timed choice's candidates are tiles, split or not, and the direct
+    forms; with a caller's also the VALU form: any of them may be chosen at
+    any rows, and the text of such a choice pins and prints unchanged."""
+    kinds = [hb.gemm_mma(K, N, 0, **TILE), hb.gemm_mma(K, N, 0, **dict(TILE, ksplit=2)),
+             hb.gemm_mm2d(K, N, 0, 32, 16).replace(mfma=16), hb.gemm_simt(K, N, 0).replace(bm=64, bn=64)]
+    for base in kinds:
+        line = gemm_line(hb, g, base, *[(32 * (i + 1), d) for i, d in enumerate(kinds) if d is not base])
+        with hb.Engine(g, "") as e:
+            e.pin(line)
+            assert e.picks() == line
+    fused = hb.gemm_mma_swiglu(K, N, **TILE)
+    line = swiglu_line(hb, g, fused, (64, hb.gemm_mma_swiglu(K, N, **dict(TILE, bm=64))))
+    with hb.Engine(g, "") as e:
+        e.pin(line)
+        assert e.picks() == line
