@@ -1492,8 +1492,10 @@ int hb_engine_picks(hb_engine* e, char* buf, uint64_t cap, uint64_t* len) {
 }
 
 // What a descriptor can be a candidate of: 1 a dense GEMM's choice, of its
-// tile, direct and VALU forms, 2 a fused gate|up's, 0 neither.
+// tile, direct and VALU forms, 2 a fused gate|up's, 0 neither (grouped rows
+// read a list and a tile table, which a dense launch does not bind).
 static int choice_of(const hb_desc& d) {
+    if (d.rows_of != HB_ROWS_DENSE) return 0;
     if (d.kind == HB_KIND_GEMM || d.kind == HB_KIND_GEMM_DIRECT || d.kind == HB_KIND_GEMM_SIMT) return 1;
     return d.kind == HB_KIND_GEMM_SWIGLU ? 2 : 0;
 }
@@ -1556,7 +1558,7 @@ int hb_engine_pin(hb_engine* e, const char* text) {
                     return bad("rows " + f[at]);
                 if (int r = kernel_at(at + 1, &v)) return r;
                 const hb_desc *a = kernel_desc(e->g, *k), *b = kernel_desc(e->g, v);
-                if (!b || choice_of(*a) != choice_of(*b) || a->k != b->k || a->n != b->n || a->out != b->out)
+                if (!b || !choice_of(*a) || choice_of(*a) != choice_of(*b) || a->k != b->k || a->n != b->n || a->out != b->out)
                     return bad(f[at + 1] + " is no kernel of this choice");
                 by_rows.push_back({rows, v});
             }

@@ -76,3 +76,20 @@ def test_text_of_every_dense_kind_reads_back(hb, g):
     with hb.Engine(g, "") as e:
         e.pin(line)
         assert e.picks() == line
+
+
+def test_text_of_other_kernels_is_refused(hb, g):
+    """A kernel that reads other operands: grouped rows (the list and the tile
+    table, which a dense launch has not), another shape or output, a fused
+    SwiGLU for a GEMM and the reverse."""
+    grouped = dict(TILE, rows_of=hb.Rows.Scatter, top_k=8, experts=64, tiles=80, rows_max=M)
+    dense = hb.gemm_mma(K, N, 0, **TILE)
+    fused = hb.gemm_mma_swiglu(K, N, **TILE)
+    for base, other in [(dense, hb.Desc(kind=hb.Kind.GEMM, k=K, n=N, out=0, **grouped)), (dense, hb.gemm_mma(K, N + 64, 0, **TILE)),
+                        (dense, hb.gemm_mma(K // 2, N, 0, **TILE)), (dense, hb.gemm_mma(K, N, hb.Out.F32, **TILE)),
+                        (dense, fused), (hb.Desc(kind=hb.Kind.GEMM, k=K, n=N, out=0, **grouped), dense)]:
+        with hb.Engine(g, "") as e, pytest.raises(hb.HerbertError, match="is no kernel of this choice"):
+            e.pin(gemm_line(hb, g, base, (64, other)))
+    for base, other in [(fused, dense), (fused, hb.gemm_mma_swiglu(K, N, **dict(grouped, rows_of=hb.Rows.Gather)))]:
+        with hb.Engine(g, "") as e, pytest.raises(hb.HerbertError, match="is no kernel of this choice"):
+            e.pin(swiglu_line(hb, g, base, (64, other)))
