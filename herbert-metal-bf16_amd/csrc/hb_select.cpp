@@ -650,17 +650,18 @@ struct hb_engine {
 
     // check_candidates (qwen.rs:2497-2545): each candidate on the full block
     // and on m - m/3 - 3 rows from a zeroed output, against candidate 0; an
-    // error beyond max|ref|/64 marks it wrong, logged, never picked.  The
-    // output and state[3] are restored.
+    // error beyond max|ref|/64 marks it wrong, logged, never picked.  state[3]
+    // is restored; the output's bytes come back in `before`, for the caller to
+    // restore once it has timed the candidates on it too.
     int check_candidates(const std::string& what, std::vector<Cand>& c,
                          std::vector<bool>& eligible, hb_range state, hb_range out,
-                         bool f32_out, uint32_t m, uint32_t row_bytes) {
+                         bool f32_out, uint32_t m, uint32_t row_bytes, std::vector<char>* before) {
         char* optr;
         uint64_t osize;
         int rc = resolve(g, out, &optr, &osize);
         if (rc) return rc;
-        std::vector<char> before(osize);
-        if ((rc = hb_download(g, out.buf, out.offset, before.data(), osize))) return rc;
+        before->resize(osize);
+        if ((rc = hb_download(g, out.buf, out.offset, before->data(), osize))) return rc;
         std::vector<std::string> wrong;
         for (uint32_t rows : {m, std::max<uint32_t>(m - m / 3 - 3, 1)}) {
             if (rows > m) rows = 1;
@@ -712,7 +713,6 @@ struct hb_engine {
                 }
             }
         }
-        if ((rc = hb_upload(g, out.buf, out.offset, before.data(), osize))) return rc;
         uint32_t st[4] = {0, 0, 0, m};
         if ((rc = hb_upload(g, state.buf, state.offset, st, 16))) return rc;
         if (!wrong.empty()) {
@@ -889,13 +889,15 @@ int hb_engine_gemm(hb_engine* e, uint32_t k, uint32_t n, uint32_t out, hb_range 
             return fail(HB_ERR_COMPILE, what + ": the production kernel mma is not built: " + hb_last_error());
     }
     uint32_t row_bytes = n * (out == HB_OUT_F32 ? 4 : 2);
-    if ((rc = e->check_candidates(what, c, eligible, state, y, out == HB_OUT_F32, m, row_bytes))) return rc;
-    size_t best;
+    std::vector<char> before;
+    size_t best = 0;
     std::vector<double> med;
     int32_t kept;
-    if ((rc = e->pick_flagged(what, c, eligible, &best, nullptr, true, &med)) ||
-        (rc = e->pick_rows(what, c, eligible, med, best, state, m, &kept)))
-        return rc;
+    if (!(rc = e->check_candidates(what, c, eligible, state, y, out == HB_OUT_F32, m, row_bytes, &before)) &&
+        !(rc = e->pick_flagged(what, c, eligible, &best, nullptr, true, &med)))
+        rc = e->pick_rows(what, c, eligible, med, best, state, m, &kept);
+    const int rc2 = before.empty() ? HB_OK : hb_upload(e->g, y.buf, y.offset, before.data(), before.size());
+    if (rc || rc2) return rc ? rc : rc2;
     e->gemm_pick[key] = kept;
     *kernel = kept;
     return HB_OK;
@@ -955,15 +957,18 @@ int hb_engine_gate_up(hb_engine* e, uint32_t h, uint32_t inter, hb_range state, 
     }
     if (c.empty()) return keep(gk, sk);
     if (fswi == 1) return c[0].name == "apart" ? keep(gk, sk) : keep(c[0].kernel, -1);
-    if ((rc = e->check_candidates(what, c, eligible, state, hout, false, m, inter * 2))) return rc;
-    size_t best;
+    std::vector<char> before;
+    size_t best = 0;
     std::vector<double> med;
-    if ((rc = e->pick_flagged(what, c, eligible, &best, nullptr, true, &med))) return rc;
+    int32_t kept = -1;
+    if (!(rc = e->check_candidates(what, c, eligible, state, hout, false, m, inter * 2, &before)) &&
+        !(rc = e->pick_flagged(what, c, eligible, &best, nullptr, true, &med)) && best != 0) {
+        eligible[0] = false;  // fewer rows take another fused form: the apart pair binds another Y
+        rc = e->pick_rows(what, c, eligible, med, best, state, m, &kept);
+    }
+    const int rc2 = before.empty() ? HB_OK : hb_upload(e->g, hout.buf, hout.offset, before.data(), before.size());
+    if (rc || rc2) return rc ? rc : rc2;
     if (best == 0) return keep(gk, sk);
-    // Fewer rows take another fused form (the apart pair binds another Y).
-    eligible[0] = eligible[0] && fswi != 2;
-    int32_t kept;
-    if ((rc = e->pick_rows(what, c, eligible, med, best, state, m, &kept))) return rc;
     return keep(kept, -1);
 }
 

@@ -145,7 +145,9 @@ hipError_t hipModuleLaunchKernel(hipFunction_t f, unsigned gx, unsigned, unsigne
                                  unsigned, hipStream_t, void** args, void**) {
     Launch l{((Fn*)f)->name, gx, 0, {}};
     clock_ms += 0.01f;
-    if (l.name != "fill_zero") {
+    if (l.name == "fill_zero") {
+        memset(*(void**)args[0], 0, *(uint64_t*)args[1]);
+    } else {
         // Kernel arguments: n pointers, then the rows.  A GEMM has 6, its
         // split's second kernel and the row kernels 3, the SwiGLU rows 2.
         const uint32_t n = l.name.rfind("gemm_splitk", 0) == 0 ? 3
