@@ -1,6 +1,6 @@
 // hb_runtime.cpp -- the HIP runtime under the C ABI: device context, buffer
 // arena, hiprtc kernel builds with an in-memory cache keyed by kernel name
-// and an on-disk code-object cache keyed by source hash, launches on the
+// and an on-disk code-object cache keyed by source and compiler, launches on the
 // context's stream and event timing.
 //
 // Reference: src/metal/gpu.rs (Gpu::open :70, alloc :150-157, pipeline
@@ -110,6 +110,22 @@ static void mkdirs(const std::string& p) {
     }
 }
 
+// The compiler that hiprtc calls reach in this process, for the cache's key.
+// A process that loaded another HIP first (PyTorch brings its own) compiles
+// with that one, whose code can be far slower (the 256 x 288 fused SwiGLU
+// tile spills there: 657 us against 163).  hiprtcVersion is 9.0 in both; the
+// runtime beside it tells them apart.
+static const std::string& compiler() {
+    static const std::string id = [] {
+        int v = 0;
+        Dl_info info;
+        if (hipRuntimeGetVersion(&v) == hipSuccess && v == HIP_VERSION) return "hiprtc" + std::to_string(v);
+        const bool known = dladdr((void*)&hiprtcCompileProgram, &info) && info.dli_fname;
+        return "hiprtc" + std::to_string(v) + " " + (known ? info.dli_fname : "");
+    }();
+    return id;
+}
+
 // Compiles `em` for `arch` with hiprtc; the code object into *code.
 static int compile(const Emitted& em, const std::string& arch, std::string* code) {
     const char* text = source_text(em.source);
@@ -127,23 +143,29 @@ static int compile(const Emitted& em, const std::string& arch, std::string* code
         if (len > 2 && strcmp(s.name + len - 2, ".h") == 0) key += s.text;
     }
     for (const auto& o : opts) key += "\n" + o;
-    key += "\nhiprtc" + std::to_string(HIP_VERSION);
-    char hex[32];
-    snprintf(hex, sizeof hex, "%016llx", (unsigned long long)fnv1a(key));
-    std::string dir = cache_dir();
-    std::string path = dir.empty() ? "" : dir + "/" + em.name + "-" + hex + ".co";
-    if (!path.empty()) {
-        std::ifstream f(path, std::ios::binary);
+    const std::string dir = cache_dir(), lib = "hiprtc" + std::to_string(HIP_VERSION), now = compiler();
+    auto entry = [&](const std::string& by) {
+        char hex[32];
+        snprintf(hex, sizeof hex, "%016llx", (unsigned long long)fnv1a(key + "\n" + by));
+        return dir.empty() ? "" : dir + "/" + em.name + "-" + hex + ".co";
+    };
+    // An entry of the compiler the library was built for is taken whichever
+    // is loaded; another's serves only processes that have that one loaded.
+    for (const std::string& by : {lib, now}) {
+        if (dir.empty()) break;
+        std::ifstream f(entry(by), std::ios::binary);
         if (f) {
             std::stringstream b;
             b << f.rdbuf();
             *code = b.str();
             if (!code->empty()) {
-                utime(path.c_str(), nullptr);  // in use: build.py keeps entries touched by its warm-up
+                utime(entry(by).c_str(), nullptr);  // in use: build.py keeps entries touched by its warm-up
                 return HB_OK;
             }
         }
+        if (by == now) break;
     }
+    const std::string path = entry(now);
     std::vector<const char*> hnames, htexts;
     for (const auto& s : kSources) {
         if (em.source == s.name) continue;
