@@ -95,9 +95,10 @@ static int emit_kind(const hb_desc& d, Emitted* e) {
                 return fail(HB_ERR_UNSUPPORTED, "gemm: tile not a multiple of waves x mfma");
             bool experts = d.rows_of != HB_ROWS_DENSE;
             // The gate and up sums meet in the LDS epilogue (dense rows,
-            // direct-to-LDS, whole 16-byte chunks of features), else in the
-            // wave's registers.
-            if (swi && (experts || !d.lds_dma || d.n % 8) && (d.bn / (d.wn * d.mfma)) % 2)
+            // direct-to-LDS, whole 16-byte chunks of features, a tile that
+            // fits there: gemm_epi.h), else in the wave's registers.
+            const bool staged = (uint64_t)d.bm * (d.bn * 2 + 16) <= 160 * 1024;
+            if (swi && (experts || !d.lds_dma || d.n % 8 || !staged) && (d.bn / (d.wn * d.mfma)) % 2)
                 return fail(HB_ERR_UNSUPPORTED,
                             "gemm_swiglu: an even count of W fragments per wave (bn / (wn * mfma))");
             if (swi && d.ksplit > 1) return fail(HB_ERR_UNSUPPORTED, "gemm_swiglu: no split K");
@@ -138,8 +139,9 @@ static int emit_kind(const hb_desc& d, Emitted* e) {
                             "8 waves (sched 1, 2) or 4 (sched 3, an even count of K tiles), whole "
                             "1 KiB loads per stage, no w_nt");
             if (d.sched &&
-                (uint64_t)(d.dbuf + 1) * (d.bm + d.bn) * d.bk * 2 > 160 * 1024)
-                return fail(HB_ERR_UNSUPPORTED, "gemm (pipelined schedules): stages beyond 160 KiB of LDS");
+                ((uint64_t)(d.dbuf + 1) * (d.bm + d.bn) * d.bk * 2 > 160 * 1024 || (swi && !staged)))
+                return fail(HB_ERR_UNSUPPORTED, "gemm (pipelined schedules): stages, or a fused SwiGLU's output "
+                                                "tile, beyond 160 KiB of LDS");
             if (d.ksplit > 16 || (d.ksplit > 1 && (swi || experts || d.k % (d.bk * d.ksplit) ||
                                                    (d.sched == 3 && (d.k / d.bk / d.ksplit) % 2))))
                 return fail(HB_ERR_UNSUPPORTED,

@@ -30,8 +30,9 @@
 // Bytes per staged tile row: the 16 bytes of padding move consecutive rows
 // four banks apart.
 constexpr u32 EPI_ROW = BN * 2 + 16;
-// Bf16 and Residual outputs whose rows are whole 16-byte chunks.
-constexpr bool EPI_LDS = OUT != 1 && N % 8 == 0 && BF % 8 == 0;
+// Bf16 and Residual outputs whose rows are whole 16-byte chunks, of tiles
+// that fit in a CU's LDS (160 KiB); others store from the registers.
+constexpr bool EPI_LDS = OUT != 1 && N % 8 == 0 && BF % 8 == 0 && BM * EPI_ROW <= 160 * 1024;
 // u32x4 of LDS the staging needs (0: direct stores).
 constexpr u32 EPI_CHUNKS = EPI_LDS ? BM * EPI_ROW / 16 : 0;
 

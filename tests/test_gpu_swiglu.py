@@ -116,6 +116,23 @@ def test_lds_fused_swiglu_equals_gemm_then_swiglu(gpu, form, m, k, nf):
     assert np.array_equal(h_fused, orc.swiglu(gu, nf))
 
 
+def test_fused_swiglu_tile_past_the_lds_epilogue(gpu):
+    """A dense fused tile whose staged output is past a CU's LDS (256 x 320):
+    its sums pair in registers, the same bits, at a ragged row tile and a
+    ragged column tile."""
+    m, k, nf = 257, 256, 296
+    x, w = inputs(m, k, nf, 0x5EED0009)
+    b = Bufs(gpu, x, w, m)
+    try:
+        b.fused(gpu.pipeline(hb.gemm_mma_swiglu(k, nf, bm=256, bn=320, bk=32, wm=4, wn=2, mfma=16, dbuf=1, lds_dma=1)), m)
+        h_fused = b.get("h")
+        b.gemm(gpu.pipeline(hb.gemm_mma(k, 2 * nf, 0, **APART)), m)
+        gu = b.get("gu")
+    finally:
+        b.free()
+    assert np.array_equal(h_fused, orc.swiglu(gu, nf))
+
+
 def test_swiglu_every_gate(gpu):
     """Every bf16 gate that is no NaN, alone among ordinary ones and beside
     its neighbours, against the oracle's exp and division, bit for bit; a NaN
