@@ -439,11 +439,15 @@ extern "C" __global__ __launch_bounds__(256) void HB_NAME(const u16* __restrict_
 // (thread t's fma chain over t, t+256, ..., the 64-lane butterfly, the 4
 // waves in order), m = ss * f32(1/D) + eps, inv = 1/sqrt(m) correctly
 // rounded, y = bf16((x * inv) * w) with w + 1 for plus_one -- the same
-// arithmetic as the matvec's fused XSrc::Norm.  The row and the weights come
-// and go in 16-byte chunks, both loaded before the sum (one memory latency);
-// the sum's order reads the row back from LDS. ----
+// arithmetic as the matvec's fused XSrc::Norm.  One memory latency bounds a
+// row of the usual lengths, so the row and the weights come and go in 16-byte
+// chunks, both loaded before the sum, whose order reads the row back from
+// LDS (2048 rows of 2560: 4.8 us against 6.6 for element loads; 1680 of
+// 79872: 171 against 272).  Rows that LDS cannot hold, past 81,900 or so
+// elements, are read from memory in each pass. ----
 static_assert(D % 256 == 0, "rmsnorm: d a multiple of 256");
 constexpr u32 CELLS = D / 8, CPT = (CELLS + 255) / 256;  // 16-byte chunks, of a thread
+constexpr bool HELD = D * 2 + 16 <= 160 * 1024;
 // A row, the weights and y may start at any element of a buffer.
 typedef u32x4 chunk_t __attribute__((aligned(2)));
 
@@ -451,30 +455,31 @@ extern "C" __global__ __launch_bounds__(256) void HB_NAME(const u16* __restrict_
                                                             const u16* __restrict__ w,
                                                             u16* __restrict__ y, u32 rows) {
     __shared__ float red[4];
-    __shared__ u32x4 row[CELLS];
+    __shared__ u32x4 row[HELD ? CELLS : 1];
     const u32 r = blockIdx.x, t = threadIdx.x, lane = t & 63u;
     if (r >= rows) return;
     const u64 base = (u64)r * D;
     const chunk_t* x4 = (const chunk_t*)(x + base);
     const chunk_t* w4 = (const chunk_t*)w;
-    u32x4 xv[CPT], wv[CPT];
+    constexpr u32 HC = HELD ? CPT : 0;
+    u32x4 xv[HELD ? CPT : 1], wv[HELD ? CPT : 1];
 #pragma unroll
-    for (u32 i = 0; i < CPT; i++) {
+    for (u32 i = 0; i < HC; i++) {
         const u32 c = t + 256 * i;
         if (CELLS % 256 == 0 || c < CELLS) xv[i] = x4[c];
     }
 #pragma unroll
-    for (u32 i = 0; i < CPT; i++) {
+    for (u32 i = 0; i < HC; i++) {
         const u32 c = t + 256 * i;
         if (CELLS % 256 == 0 || c < CELLS) wv[i] = w4[c];
     }
 #pragma unroll
-    for (u32 i = 0; i < CPT; i++) {
+    for (u32 i = 0; i < HC; i++) {
         const u32 c = t + 256 * i;
         if (CELLS % 256 == 0 || c < CELLS) row[c] = xv[i];
     }
-    __syncthreads();
-    const u16* xs = (const u16*)row;
+    if constexpr (HELD) __syncthreads();
+    const u16* xs = HELD ? (const u16*)row : x + base;
     float a = 0.0f;
 #pragma unroll
     for (u32 i = 0; i < D / 256; i++) {
@@ -491,15 +496,16 @@ extern "C" __global__ __launch_bounds__(256) void HB_NAME(const u16* __restrict_
     for (u32 i = 0; i < CPT; i++) {
         const u32 c = t + 256 * i;
         if (CELLS % 256 != 0 && c >= CELLS) break;
+        const u32x4 xc = HELD ? xv[HELD ? i : 0] : (u32x4)x4[c], wc = HELD ? wv[HELD ? i : 0] : (u32x4)w4[c];
         u32x4 o;
 #pragma unroll
         for (u32 e = 0; e < 4; e++) {
-            float w0 = bf16_lo(wv[i][e]), w1 = bf16_hi(wv[i][e]);
+            float w0 = bf16_lo(wc[e]), w1 = bf16_hi(wc[e]);
             if (HB_PLUS1) {
                 w0 = w0 + 1.0f;
                 w1 = w1 + 1.0f;
             }
-            o[e] = pack_bf16x2((bf16_lo(xv[i][e]) * inv) * w0, (bf16_hi(xv[i][e]) * inv) * w1);
+            o[e] = pack_bf16x2((bf16_lo(xc[e]) * inv) * w0, (bf16_hi(xc[e]) * inv) * w1);
         }
         ((chunk_t*)(y + base))[c] = o;
     }

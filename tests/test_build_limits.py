@@ -28,3 +28,9 @@ def test_fused_swiglu_tiles_that_pair_nowhere(monkeypatch):
     with pytest.raises(hb.HerbertError, match="output tile, beyond 160 KiB"):
         precompile(hb.gemm_mma_swiglu(256, 512, bm=256, bn=320, bk=32, wm=4, wn=2, mfma=16, dbuf=3, lds_dma=1, sched=1),
                    monkeypatch)
+
+
+@pytest.mark.parametrize("d", [81664, 81920, 262144])
+def test_rmsnorm_rows_past_lds(monkeypatch, d):
+    """Rows that LDS holds, and longer ones, which it does not."""
+    precompile(hb.rmsnorm(d, 1e-6, True), monkeypatch)

@@ -196,10 +196,11 @@ def test_moe_layer_through_picked_kernels(gpu):
     gpu.free(Wdn)
 
 
-@pytest.mark.parametrize("d,rows,at", [(256, 3, 0), (2304, 5, 1), (2560, 2, 7)])
+@pytest.mark.parametrize("d,rows,at", [(256, 3, 0), (2304, 5, 1), (2560, 2, 7), (81664, 2, 1), (81920, 2, 3)])
 def test_rmsnorm_any_start(gpu, d, rows, at):
     """Rows, weights and outputs that start `at` elements into their buffers
-    (2-byte aligned only), one chunk a row of threads and ragged counts."""
+    (2-byte aligned only), one chunk a row of threads and ragged counts; the
+    longest row that LDS holds and the first that it does not."""
     x = hb.normal_bf16(53, 2.0, (at + rows * d,))
     w = hb.normal_bf16(54, 0.1, (at + d,))
     X, Wb, Y = gpu.alloc_with(x), gpu.alloc_with(w), gpu.alloc_with(np.full(at + rows * d + 3, 0x7FC1, np.uint16))
