@@ -63,31 +63,33 @@ HB_DEV float hb_expf(float x) {
 // src/msl/mod.rs:885-890: 1 / (1 + e^-x), an IEEE division.
 HB_DEV float hb_sigmoid(float x) { return 1.0f / (1.0f + hb_expf(-x)); }
 
-// h[i] = (g[i] * sigmoid(g[i])) * u[i] for n bf16-valued gates: the bits of
-// hb_sigmoid on all 65536 of them, in 25 instructions an output against 40
-// (a 256 x 288 tile's SwiGLU took 7 us of VALU issue).  While no gate is
-// below -87, e^-g <= 2^126 and needs no upper range check; the lower one is
-// a clamp (past it 1 + e^-g is 1); and the division is v_rcp_f32 with one
+// (g * sigmoid(g)) * u.  A NaN gate gives sigmoid's NaN (-g, quiet), which
+// with two NaN factors would be the compiler's choice of their order.
+HB_DEV float swiglu_f(float g, float u) {
+    const float s = hb_sigmoid(g);
+    return g != g ? s : (g * s) * u;
+}
+
+// swiglu_f of n bf16-valued gates: its bits on all 65536 of them, in 24
+// instructions an output against 40 (a 256 x 288 tile's SwiGLU took 7 us of
+// VALU issue).  While every gate is within +-87, e^-g is within 2^-126 and
+// 2^126 and needs no range checks, and the division is v_rcp_f32 with one
 // Newton step by fma (Markstein), which equals the IEEE quotient for every
 // float d from 1 to 2^126 (all 1.06e9 compared).  One test covers the n
-// gates: as unsigned words, the most negative is the largest.  A NaN gate
-// gives a NaN either way.
+// gates; a NaN is not within the range.
 template <u32 n>
 HB_DEV void swiglu_n(const float* g, const float* u, float* h) {
-    u32 top = 0;
+    bool near = true;
 #pragma unroll
-    for (u32 i = 0; i < n; i++) {
-        const u32 b = __builtin_bit_cast(u32, g[i]);
-        top = b > top ? b : top;
-    }
-    if (top > 0xc2ae0000u) {  // below -87, or a negative NaN
+    for (u32 i = 0; i < n; i++) near &= __builtin_fabsf(g[i]) <= 87.0f;
+    if (!near) {
 #pragma unroll 1
-        for (u32 i = 0; i < n; i++) h[i] = (g[i] * hb_sigmoid(g[i])) * u[i];
+        for (u32 i = 0; i < n; i++) h[i] = swiglu_f(g[i], u[i]);
         return;
     }
 #pragma unroll
     for (u32 i = 0; i < n; i++) {
-        const float d = 1.0f + exp_core(__builtin_amdgcn_fmed3f(-g[i], -104.0f, 104.0f));
+        const float d = 1.0f + exp_core(-g[i]);
         const float r = __builtin_amdgcn_rcpf(d);
         h[i] = (g[i] * __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r)) * u[i];
     }

@@ -125,7 +125,7 @@ static_assert(HB_FORM != 4 || (MV <= 8 && KS % 128 == 0 && HB_XSRC == 0 && !SWO 
 
 // bf16(g * sigmoid(g) * u) as f32: swiglu's arithmetic (the SwiGLU kernels'
 // own expression, kernels.rs:256-261).
-HB_DEV float swiglu1(float g, float u) { return round_bf16((g * hb_sigmoid(g)) * u); }
+HB_DEV float swiglu1(float g, float u) { return round_bf16(swiglu_f(g, u)); }
 
 HB_DEV void store_out(void* y, u64 at, float v) {
     if constexpr (OUT == 1) {

@@ -160,6 +160,27 @@ def test_swiglu_every_gate(gpu):
             assert np.all((got[bad] & 0x7FFF) > 0x7F80)
 
 
+def test_swiglu_nan_gates(gpu):
+    """A NaN gate gives its sigmoid's NaN whatever u is: -g, quiet, as the
+    oracle's does; alone in its 16 bytes and beside other gates."""
+    nans = np.arange(65536, dtype=np.uint32).astype(np.uint16)
+    nans = nans[(nans & 0x7FFF) > 0x7F80]
+    want = (nans ^ 0x8000) | 0x0040
+    ks = gpu.pipeline(hb.swiglu_rows(8))
+    for u in (0x3F80, 0x0000, 0x7F80, 0x7FC1, 0xFFA5):
+        gu = np.full((len(nans), 16), u, np.uint16)
+        gu[:, :8] = 0x3F80
+        gu[:, 3] = gu[:, 6] = nans
+        a, h = gpu.alloc_with(gu), gpu.alloc(gu.nbytes // 2)
+        try:
+            gpu.launch(ks, [hb.r(a), hb.r(h)], len(nans))
+            got = gpu.download(h, np.uint16, gu.size // 2).reshape(-1, 8)
+        finally:
+            gpu.free(a)
+            gpu.free(h)
+        assert np.array_equal(got[:, 3], want) and np.array_equal(got[:, 6], want), hex(u)
+
+
 def test_fused_swiglu_state_rows(gpu):
     """state[3] below the launch's rows: only state[3] rows of h written."""
     m, k, nf = 256, 256, 512
