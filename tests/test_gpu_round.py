@@ -1,10 +1,11 @@
 """The rounding probe of herbert-metal-probe `round`
 (src/bin/herbert-metal-probe.rs:7-11): every f32 bit pattern, in 256 chunks
-of 2^24, rounded to bf16 on the GPU by the integer form every epilogue uses,
+of 2^24, rounded to bf16 on the GPU by the integer form of the single stores,
 compared with the CPU oracle's f32_to_bf16 (src/core/bf16.rs:13-23) and the
-differences counted by class of the input.  The compiler's own conversion
-(gfx950 v_cvt_pk_bf16_f32) is probed the same way: it must agree on every
-non-NaN pattern (NaN payloads may differ; they are counted, not required)."""
+differences counted by class of the input.  The conversion of the paired
+stores (gfx950 v_cvt_pk_bf16_f32) is probed the same way: it must agree on
+every non-NaN pattern (NaN payloads may differ here, where f32 NaNs of any
+payload go in; they are counted, not required)."""
 import numpy as np
 import pytest
 
