@@ -651,8 +651,9 @@ struct hb_engine {
     // check_candidates (qwen.rs:2497-2545): each candidate on the full block
     // and on m - m/3 - 3 rows from a zeroed output, against candidate 0; an
     // error beyond max|ref|/64 marks it wrong, logged, never picked.  state[3]
-    // is restored; the output's bytes come back in `before`, for the caller to
-    // restore once it has timed the candidates on it too.
+    // is restored; the output's bytes come back in `before` (empty where they
+    // could not be read, and nothing ran), for the caller to restore once it
+    // has timed the candidates on it too.
     int check_candidates(const std::string& what, std::vector<Cand>& c,
                          std::vector<bool>& eligible, hb_range state, hb_range out,
                          bool f32_out, uint32_t m, uint32_t row_bytes, std::vector<char>* before) {
@@ -660,8 +661,9 @@ struct hb_engine {
         uint64_t osize;
         int rc = resolve(g, out, &optr, &osize);
         if (rc) return rc;
-        before->resize(osize);
-        if ((rc = hb_download(g, out.buf, out.offset, before->data(), osize))) return rc;
+        std::vector<char> now(osize);
+        if ((rc = hb_download(g, out.buf, out.offset, now.data(), osize))) return rc;
+        before->swap(now);
         std::vector<std::string> wrong;
         for (uint32_t rows : {m, std::max<uint32_t>(m - m / 3 - 3, 1)}) {
             if (rows > m) rows = 1;

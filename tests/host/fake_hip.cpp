@@ -22,7 +22,7 @@ struct Launch {
     std::vector<void*> ptrs;
 };
 std::map<void*, size_t> blocks;
-uint64_t in_use = 0, limit = ~0ull, tries = 0;
+uint64_t in_use = 0, limit = ~0ull, tries = 0, failing_reads = 0;
 std::vector<Launch> launches;
 float clock_ms = 0;  // 10 us a launch
 struct Fn {
@@ -35,6 +35,8 @@ extern "C" {
 
 // ---- what a test reads and sets ----
 void fake_limit(uint64_t bytes) { limit = bytes; }
+// The next n copies to the host fail.
+void fake_fail_reads(uint64_t n) { failing_reads = n; }
 uint64_t fake_in_use(void) { return in_use; }
 uint64_t fake_malloc_tries(void) { return tries; }
 void fake_forget(void) { launches.clear(); }
@@ -71,7 +73,11 @@ hipError_t hipFree(void* p) {
     free(p);
     return hipSuccess;
 }
-hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind kind, hipStream_t) {
+    if (kind == hipMemcpyDeviceToHost && failing_reads) {
+        failing_reads--;
+        return hipErrorUnknown;
+    }
     memcpy(d, s, n);
     return hipSuccess;
 }

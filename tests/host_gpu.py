@@ -48,7 +48,7 @@ def load(out):
     spec.loader.exec_module(hb)
     for name in ("fake_in_use", "fake_malloc_tries", "fake_launch_span"):
         getattr(hb.lib, name).restype = ctypes.c_uint64
-    hb.lib.fake_limit.argtypes = [ctypes.c_uint64]
+    hb.lib.fake_limit.argtypes = hb.lib.fake_fail_reads.argtypes = [ctypes.c_uint64]
     hb.lib.fake_launch_name.restype = ctypes.c_char_p
     hb.lib.fake_launches.restype = hb.lib.fake_launch_rows.restype = ctypes.c_uint32
     return hb

@@ -35,3 +35,22 @@ def test_choice_restores_its_output(hb):
         assert g.download(st, np.uint32, 4)[3] == M
     finally:
         g.close()
+
+
+def test_output_that_cannot_be_read_stays(hb):
+    """A choice that could not read Y before its runs fails and writes none
+    of it."""
+    g = hb.Gpu(0)
+    try:
+        st = g.alloc_with(np.array([7, 8, 9, M], np.uint32))
+        w, x = g.alloc(N * K * 2), g.alloc(M * K * 2)
+        y0 = np.arange(1, M * N + 1, dtype=np.uint16)
+        y = g.alloc_with(y0)
+        with hb.Engine(g, "") as e:
+            hb.lib.fake_fail_reads(1)
+            with pytest.raises(hb.HerbertError):
+                e.gemm(K, N, hb.Out.Residual, hb.r(st), hb.r(w), hb.r(x), hb.r(y), M)
+        hb.lib.fake_fail_reads(0)
+        assert np.array_equal(g.download(y, np.uint16, M * N), y0)
+    finally:
+        g.close()
