@@ -247,7 +247,7 @@ const Form kForms[10] = {
     {"mma_t64", 64, 64, 32, 1, 4, 16, 0, 0, 0},
 };
 // Timed with the table but not named by gemm.mform: tiles whose counts
-// fill whole rounds of the 256 CUs on this build's shapes (256 x 192:
+// fill whole rounds of the 256 CUs on the 4B-class shapes (256 x 192:
 // 768 tiles at 2048 x 18432; 128 x 160: 256 at 2048 x 2560; 128 x 192:
 // 224 at 2048 x 2560, 8 wavefronts), three and four stages of 64 K for the
 // long-K shapes, and the band tile order of gemm_nax (prefill.rs:615-631):
@@ -286,9 +286,13 @@ const Form kMoreForms[] = {
     {"mma_t64x64_s4", 64, 64, 64, 4, 1, 16, 3, 1, 1},
     {"mma_t32x96_k128_s4", 32, 96, 128, 2, 2, 16, 3, 1, 1},
     {"mma_t128x80_s3", 128, 80, 64, 2, 1, 16, 2, 1, 1},
-    // Row tiles of 192 for the row counts between those of 128 and 256.
+    // Row tiles of 192, for the row counts where they run one round of the CUs
+    // and tiles of 128 rows two: 1280 rows of 17408 x 5120 235 us against 297
+    // by 256 x 160 and 329 by 128 x 192, 576 of 2560 x 10240 44.7 against 51.1
+    // and 58.4 (cold).  Where 128 rows make one round too these are the
+    // faster (1100 rows: 201 against 229).  The ping-pong schedule of this
+    // tile was 7-28% slower at each of 37 shapes and row counts, so is none.
     {"mma_t192x160_w8_s3", 192, 160, 64, 4, 2, 16, 2, 1, 1},
-    {"pp_t192x160_k64", 192, 160, 64, 4, 2, 16, 2, 1, 1, 0, 1},
     // Eight waves in two groups taking turns between memory and MFMA phases
     // (hb_desc.sched 1), four stages of 32 K: 256 x 288 tiles fill exactly
     // two rounds of the CUs on 2048 x 18432 (and 4608: 128 tiles).
@@ -345,7 +349,9 @@ const Form kSplitForms[] = {
 // narrow last ones are for short prompts, one row tile of 64 or 128 rows:
 // enough column tiles to reach every CU (230 of 80 W rows at 2 x 9216), and
 // 128 K a stage so that each barrier covers twice the loads (64 rows: 23.3 us
-// against 27.6 for the best unfused form and its pass).
+// against 27.6 for the best unfused form and its pass).  Row tiles of 192 as
+// among the dense forms: 330 rows 47.7 us (cold) against 56.2 by 256 x 80 and
+// 67.1 by 128 x 80; their ping-pong schedule 1-20% slower at each of 19.
 const Form kFusedForms[] = {
     {"fused128x64", 128, 128, 64, 2, 2, 16, 1, 1, 1},
     {"fused128x64b2", 128, 128, 64, 2, 2, 16, 1, 1, 0, 2},
@@ -358,7 +364,6 @@ const Form kFusedForms[] = {
     {"fused256x80_pp_b4", 256, 160, 64, 4, 2, 16, 2, 1, 1, 4, 1},
     {"fused128x80_pp", 128, 160, 64, 4, 2, 16, 3, 1, 1, 0, 1},
     {"fused192x80_w8_s3", 192, 160, 64, 4, 2, 16, 2, 1, 1},
-    {"fused192x80_pp", 192, 160, 64, 4, 2, 16, 2, 1, 1, 0, 1},
     {"fused128x96_w8_s4", 128, 192, 64, 2, 4, 16, 3, 1, 0},
     {"fused128x80_s4", 128, 160, 64, 4, 1, 16, 3, 1, 1},
     {"fused128x40_s4", 128, 80, 64, 4, 1, 16, 3, 1, 1},
