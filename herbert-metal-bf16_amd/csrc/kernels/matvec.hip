@@ -6,7 +6,7 @@
 // rows, lanes striding K by 8 bf16, an fma chain per lane, the simdgroup
 // sum), :502-519 and :640-975 (matvec_split: `split` simdgroups sharing a
 // row's K, partials folded in simdgroup order, persistent groups), :223-236
-// (store).  The reference decodes one row; m up to MV_M is this build's
+// (store).  The reference decodes one row; m up to MV_M is this library's
 // extension (one W read serves every row).
 //
 // Four forms (HB_FORM):
@@ -227,6 +227,8 @@ extern "C" __global__ __launch_bounds__(NT) void HB_NAME(const u16* __restrict__
 #pragma unroll
         for (u32 j = 0; j < MV; j++) {
             float a = 0.0f;
+            // Ten LDS reads in flight: a row of 2560 at once, a longer one in
+            // turns of ten and the rest (each row's adds are one chain).
 #pragma unroll 10
             for (u32 i = 0; i < K / 256; i++) {
                 const float v = bf16_to_f32(xs[j * K + tid + i * 256]);

@@ -301,7 +301,11 @@ int hb_engine_buckets(hb_engine *engine, uint32_t *out, uint32_t cap, uint32_t *
  * A timed choice also times its best candidates at fewer rows (5/8, 3/4 and
  * 7/8 of m): *kernel launched over m' rows runs the one kept for m', with
  * the same bindings; its name and kind are those of m.  Its first launch
- * sizes the split-K workspace for every row count up to m. */
+ * sizes the split-K workspace for every row count up to m.  A row's low bits
+ * (the order of its f32 sums) so depend on how many rows the launch has, and,
+ * where the workspace cannot grow (a recorded graph holds it, or memory ran
+ * out), rows whose kernel needs more of it run the kernel of m.  Launches of
+ * one row count in one state of the workspace give the same bits. */
 int hb_engine_gemm(hb_engine *engine, uint32_t k, uint32_t n, uint32_t out, hb_range state,
                    hb_range w, hb_range x, hb_range y, uint32_t m, int32_t *kernel);
 
@@ -430,7 +434,9 @@ int hb_engine_picks(hb_engine *engine, char *buf, uint64_t cap, uint64_t *len);
 /* Seeds the engine's choices with text hb_engine_picks wrote (on this or
  * another process or box): each kernel is built from its descriptor and
  * must come out under the recorded name; later selections of those keys
- * return them without timing.  HB_ERR_INVALID naming the line otherwise. */
+ * return them without timing.  Choices at fewer rows: dense kernels of the
+ * choice's shape, rows ascending, none past those of the key.
+ * HB_ERR_INVALID naming the line otherwise. */
 int hb_engine_pin(hb_engine *engine, const char *text);
 /* One more candidate for the engine's next GEMM choices, after the built-in
  * ones (the way check_candidates meets a kernel that builds but computes
