@@ -1595,7 +1595,8 @@ int hb_engine_pin(hb_engine* e, const char* text) {
         } else if (f[0] == "experts") {
             if (f.size() < 11) return bad("too few fields");
             hb_engine::ExpertsPick ep;
-            ep.bm = (uint32_t)std::stoul(f[2]);
+            std::string err;
+            if (!Tune::parse_u32(f[2], &ep.bm, &err)) return bad("rows " + f[2]);
             for (int i = 0; i < 4; i++)
                 if ((rc = kernel_at(3 + 2 * i, &ep.kernels[i]))) return rc;
             e->experts_pick[f[1]] = ep;

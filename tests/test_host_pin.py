@@ -93,3 +93,12 @@ def test_text_of_other_kernels_is_refused(hb, g):
     for base, other in [(fused, dense), (fused, hb.gemm_mma_swiglu(K, N, **dict(grouped, rows_of=hb.Rows.Gather)))]:
         with hb.Engine(g, "") as e, pytest.raises(hb.HerbertError, match="is no kernel of this choice"):
             e.pin(swiglu_line(hb, g, base, (64, other)))
+
+
+@pytest.mark.parametrize("rows", ["", "x", "99999999999999999999999"])
+def test_experts_line_without_tile_rows_is_refused(hb, g, rows):
+    """An experts line whose tile rows are no number is an error like any
+    other line's."""
+    line = "experts\tkey\t%s\t" % rows + "\t".join(["-", "-"] * 4) + "\n"
+    with hb.Engine(g, "") as e, pytest.raises(hb.HerbertError, match="line 1: rows"):
+        e.pin(line)
